@@ -744,10 +744,20 @@ struct vk_reranker {
     hipStream_t stream = nullptr;
     DeviceBuffer<float> base, queries;
     DeviceBuffer<Pair> candidates, out;
-    DeviceBuffer<unsigned> error;
+    PinnedBuffer<unsigned> error;  // written by the kernel (host memory) when a candidate id is >= n
+    bool in_flight = false;        // a call raised before its stream completed: its kernel may still write `error`
+    std::unique_ptr<StageClock> clock_pool;
 
     ~vk_reranker() {
+        clock_pool.reset();  // its events before the stream
         if (stream) (void)hipStreamDestroy(stream);
+    }
+
+    // The stage clock of this re-ranker's calls: its events are created once and reused by every call.
+    StageClock& stage_clock() {
+        if (!clock_pool) clock_pool = std::make_unique<StageClock>(stream);
+        clock_pool->reset();
+        return *clock_pool;
     }
 
     static void check(size_t r, size_t k) {
@@ -759,7 +769,9 @@ struct vk_reranker {
     void run(const float* d_q, size_t nq, const Pair* d_c, size_t r, size_t k, Pair* d_o, vk_timings* t,
              StageClock& clock) {
         error.ensure(1);
-        VK_HIP(hipMemsetAsync(error.get(), 0, sizeof(unsigned), stream));
+        if (in_flight) VK_HIP(hipStreamSynchronize(stream));
+        *error.get() = 0;
+        in_flight = true;
         vk::RerankArgs a{};
         a.base = base.get();
         a.n = static_cast<int64_t>(n);
@@ -776,16 +788,15 @@ struct vk_reranker {
     }
 
     void finish(StageClock& clock) {
-        unsigned flag = 0;
-        VK_HIP(hipMemcpyAsync(&flag, error.get(), sizeof flag, hipMemcpyDeviceToHost, stream));
         clock.settle();
-        if (flag) fail(VK_ERR_INVALID_ARGUMENT, "a candidate id is >= n (the number of base vectors)");
+        in_flight = false;
+        if (*error.get()) fail(VK_ERR_INVALID_ARGUMENT, "a candidate id is >= n (the number of base vectors)");
     }
 
     void rerank_host(const float* host_q, size_t nq, const vk_neighbor* host_c, size_t r, size_t k,
                      vk_neighbor* host_o, vk_timings* t) {
         VK_HIP(hipSetDevice(device));
-        StageClock clock(stream);
+        StageClock& clock = stage_clock();
         queries.ensure(nq * d);
         candidates.ensure(nq * r);
         out.ensure(nq * k);
@@ -803,7 +814,7 @@ struct vk_reranker {
     void rerank_device(const float* d_q, size_t nq, const vk_neighbor* d_c, size_t r, size_t k, vk_neighbor* d_o,
                        vk_timings* t) {
         VK_HIP(hipSetDevice(device));
-        StageClock clock(stream);
+        StageClock& clock = stage_clock();
         run(d_q, nq, reinterpret_cast<const Pair*>(d_c), r, k, reinterpret_cast<Pair*>(d_o), t, clock);
         finish(clock);
     }
@@ -1069,9 +1080,18 @@ struct vk_ivf {
     PinnedBuffer<float> staged_q;  // host-buffer searches: queries and results staged in page-locked memory
     PinnedBuffer<Pair> staged_out;
     std::vector<int64_t> list_tile_h;  // [nlist + 1]
+    std::unique_ptr<StageClock> clock_pool;
 
     ~vk_ivf() {
+        clock_pool.reset();  // its events before the stream
         if (stream) (void)hipStreamDestroy(stream);
+    }
+
+    // The stage clock of this index's calls: its events are created once and reused by every call.
+    StageClock& stage_clock() {
+        if (!clock_pool) clock_pool = std::make_unique<StageClock>(stream);
+        clock_pool->reset();
+        return *clock_pool;
     }
 
     void check(size_t nprobe, size_t k) const {
@@ -1293,7 +1313,7 @@ VK_EXPORT int vk_ivf_search(vk_ivf* v, const float* queries, size_t nq, size_t n
         if (nq > 0) {
             require(queries != nullptr && out != nullptr, "queries and out must not be null");
             VK_HIP(hipSetDevice(v->device));
-            StageClock clock(v->stream);
+            StageClock& clock = v->stage_clock();
             const size_t batch = 16384;  // queries per batch: the table kernel's grid and the per-search buffers
             for (size_t q0 = 0; q0 < nq; q0 += batch) {
                 const size_t b = std::min(batch, nq - q0);
@@ -1328,7 +1348,7 @@ VK_EXPORT int vk_ivf_search_device(vk_ivf* v, const float* d_queries, size_t nq,
         if (nq > 0) {
             require(d_queries != nullptr && d_out != nullptr, "queries and out must not be null");
             VK_HIP(hipSetDevice(v->device));
-            StageClock clock(v->stream);
+            StageClock& clock = v->stage_clock();
             const size_t batch = 16384;  // queries per batch, as in vk_ivf_search
             for (size_t q0 = 0; q0 < nq; q0 += batch) {
                 const size_t b = std::min(batch, nq - q0);
