@@ -26,10 +26,12 @@ namespace vk {
 // Per-m instance tables of the wave-list scan, fp32 (fused_wave_m*.hip) and fp16 tables (fused_wave_h*.hip).
 WaveScanKernel fused_wave_kernel_m16(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_m32(int qg, int ng, int ilp, int segments, bool bulk, int threads);
+WaveScanKernel fused_wave_kernel_m48(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_m64(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_mx(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_h16(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_h32(int qg, int ng, int ilp, int segments, bool bulk, int threads);
+WaveScanKernel fused_wave_kernel_h48(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_h64(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_hx(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 
@@ -38,6 +40,7 @@ WaveScanKernel fused_wave_kernel(int qg, int ng, int ilp, int m, int segments, b
         switch (m) {
             case 16: return fused_wave_kernel_h16(qg, ng, ilp, segments, bulk, threads);
             case 32: return fused_wave_kernel_h32(qg, ng, ilp, segments, bulk, threads);
+            case 48: return fused_wave_kernel_h48(qg, ng, ilp, segments, bulk, threads);
             case 64: return fused_wave_kernel_h64(qg, ng, ilp, segments, bulk, threads);
             default: return fused_wave_kernel_hx(qg, ng, ilp, segments, bulk, threads);
         }
@@ -45,6 +48,7 @@ WaveScanKernel fused_wave_kernel(int qg, int ng, int ilp, int m, int segments, b
     switch (m) {
         case 16: return fused_wave_kernel_m16(qg, ng, ilp, segments, bulk, threads);
         case 32: return fused_wave_kernel_m32(qg, ng, ilp, segments, bulk, threads);
+        case 48: return fused_wave_kernel_m48(qg, ng, ilp, segments, bulk, threads);
         case 64: return fused_wave_kernel_m64(qg, ng, ilp, segments, bulk, threads);
         default: return fused_wave_kernel_mx(qg, ng, ilp, segments, bulk, threads);
     }
@@ -1074,9 +1078,11 @@ struct vk_ivf {
     hipStream_t stream = nullptr;
     DeviceBuffer<float> coarse, centroids, queries, lut, coarse_dist;
     DeviceBuffer<uint4> codes_v;
-    DeviceBuffer<int32_t> ids, slab_queries;
+    DeviceBuffer<int32_t> ids;
     DeviceBuffer<int64_t> list_tile, slab_tile, slab_gran, query_gran;
-    DeviceBuffer<Pair> probes, part, out;
+    DeviceBuffer<unsigned> plan_ticket;
+    bool ticket_clean = false;  // false until zeroed, and after a search that stopped before its stream completed
+    DeviceBuffer<Pair> part, out;
     PinnedBuffer<float> staged_q;  // host-buffer searches: queries and results staged in page-locked memory
     PinnedBuffer<Pair> staged_out;
     std::vector<int64_t> list_tile_h;  // [nlist + 1]
@@ -1105,7 +1111,6 @@ struct vk_ivf {
         // 1. the nprobe nearest lists of every query: exact distances to all coarse centroids (a dense tile
         // kernel), then the nprobe smallest of each row by (dist, list id); in row chunks that keep the distance
         // matrix within 64 Mi floats
-        probes.ensure(nq * nprobe);
         const size_t rows = std::max<size_t>(1, std::min(nq, (size_t{64} << 20) / nlist));
         coarse_dist.ensure(rows * nlist);
         lut.ensure(nq * m * vk::KSUB);
@@ -1113,29 +1118,34 @@ struct vk_ivf {
         // so a query's slabs are one run of consecutive granules
         const size_t slabs = nq * nprobe;
         slab_tile.ensure(slabs);
-        slab_queries.ensure(slabs);
-        slab_gran.ensure(slabs + 1);
+        slab_gran.ensure(slabs);
         query_gran.ensure(nq + 1);
-        vk::IvfPlanArgs plan{probes.get(),      static_cast<int>(nprobe), static_cast<int64_t>(nq), list_tile.get(),
-                             slab_tile.get(),   slab_queries.get(),       slab_gran.get(),           query_gran.get()};
+        plan_ticket.ensure(1);
+        if (!ticket_clean) VK_HIP(vk::launch_zero_words(plan_ticket.get(), 1, stream));
+        ticket_clean = false;  // until the stream has completed this search
         clock.time(&t->lut_ms, [&] {
             for (size_t r0 = 0; r0 < nq; r0 += rows) {
                 const size_t nr = std::min(rows, nq - r0);
+                // the tables of every query come with the first rows' distances
+                const vk::ProbeLut tables{r0 == 0 ? d_q : nullptr, centroids.get(), static_cast<int>(m),
+                                          static_cast<int>(nq), lut.get()};
                 VK_HIP(vk::launch_coarse_distances(d_q + r0 * d, static_cast<int64_t>(nr), coarse.get(),
                                                    static_cast<int64_t>(nlist), static_cast<int>(d), coarse_dist.get(),
-                                                   stream));
-                vk::SelectArgs sel{};
-                sel.mode = 0;
-                sel.dists = coarse_dist.get();
-                sel.len = static_cast<int64_t>(nlist);
-                sel.K = vk::plan::dispatched_k(nprobe);
-                sel.k = static_cast<int>(nprobe);
-                sel.out = probes.get() + r0 * nprobe;
-                VK_HIP(vk::launch_select(sel, static_cast<int>(nr), stream));
+                                                   tables, stream));
+                vk::IvfPlanArgs plan{};
+                plan.dists = coarse_dist.get();
+                plan.nlist = static_cast<int64_t>(nlist);
+                plan.first = static_cast<int64_t>(r0);
+                plan.K = vk::plan::dispatched_k(nprobe);
+                plan.nprobe = static_cast<int>(nprobe);
+                plan.nq = static_cast<int64_t>(nq);
+                plan.list_tile = list_tile.get();
+                plan.slab_tile = slab_tile.get();
+                plan.slab_gran = slab_gran.get();
+                plan.query_gran = query_gran.get();
+                plan.ticket = plan_ticket.get();
+                VK_HIP(vk::launch_ivf_plan(plan, static_cast<int>(nr), stream));
             }
-            VK_HIP(vk::launch_lut(d_q, centroids.get(), static_cast<int>(d), static_cast<int>(m), static_cast<int>(nq),
-                                  1, static_cast<int>(nq), lut.get(), stream));
-            VK_HIP(vk::launch_ivf_plan(plan, stream));
         });
 
         // 3. the scan over the probed lists: a balanced partition of all granules over one wave of blocks (the
@@ -1176,10 +1186,9 @@ struct vk_ivf {
         a.k = static_cast<int>(kk);
         a.lists_per_block = W;
         a.part = part.get();
-        a.n_slabs = static_cast<int64_t>(slabs);
+        a.nprobe = static_cast<int>(nprobe);
         a.slab_gran = slab_gran.get();
         a.slab_tile = slab_tile.get();
-        a.slab_queries = slab_queries.get();
         a.query_gran = query_gran.get();
         a.list_tile = list_tile.get();
         a.ids = ids.get();
@@ -1332,6 +1341,7 @@ VK_EXPORT int vk_ivf_search(vk_ivf* v, const float* queries, size_t nq, size_t n
                                           hipMemcpyDeviceToHost, v->stream));
                 });
                 clock.settle();
+                v->ticket_clean = true;
                 std::memcpy(out + q0 * k, v->staged_out.get(), b * k * sizeof(Pair));
             }
         }
@@ -1354,6 +1364,7 @@ VK_EXPORT int vk_ivf_search_device(vk_ivf* v, const float* d_queries, size_t nq,
                 const size_t b = std::min(batch, nq - q0);
                 v->search(d_queries + q0 * v->d, b, nprobe, k, reinterpret_cast<Pair*>(d_out) + q0 * k, &t, clock);
                 clock.settle();
+                v->ticket_clean = true;
             }
         }
         if (timings) *timings = t;

@@ -7,6 +7,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 namespace vk {
 
@@ -416,6 +417,45 @@ __device__ __forceinline__ void stream_partials(WaveList<S, true>& wl, const Pai
                                                 int lists, int K, int lane) {
     if (K > 32) stream_lists(wl, first, part, parts, lists, K, lane);
     else stream_pairs(wl, first, part * 4 * WAVE, parts * 4 * WAVE, lists * K, K, lane);
+}
+
+// Streams wave `wave`'s share of a row of distances (ids are column indices) through its list, W waves in all.
+// Long rows (n distances of an unfused scan): each wave reads 4 x 1 KB per round (16-byte loads, four in flight) and
+// offers them as 16 candidates per lane; the threshold test rejects nearly all of them once the list fills. Short
+// rows (an IVF probe's nlist distances): one 16-byte load per lane per round, so that every wave of the block takes
+// a share of the row.
+template <int S, int W>
+__device__ __forceinline__ void stream_row(WaveList<S, true>& list, const float* row, int64_t len, int K, int wave,
+                                           int lane) {
+    constexpr int V = 4;
+    const bool vec = len % V == 0 && reinterpret_cast<uintptr_t>(row) % 16 == 0;
+    auto rounds = [&](auto r_tag) -> int64_t {
+        constexpr int R = decltype(r_tag)::value, CH = WAVE * V * R;  // floats per wave per round
+        const int64_t full = vec ? len / CH * CH : 0;  // complete rounds; chunk c goes to wave c % W
+        for (int64_t base = static_cast<int64_t>(wave) * CH; base < full; base += W * CH) {
+            float4 v[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[r] = *reinterpret_cast<const float4*>(row + base + (r * WAVE + lane) * V);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int32_t j = static_cast<int32_t>(base + (r * WAVE + lane) * V);
+                list.offer(v[r].x, j, true, K);
+                list.offer(v[r].y, j + 1, true, K);
+                list.offer(v[r].z, j + 2, true, K);
+                list.offer(v[r].w, j + 3, true, K);
+            }
+        }
+        return full;
+    };
+    const int64_t full = len >= int64_t{W} * WAVE * V * 4 ? rounds(std::integral_constant<int, 4>{})
+                                                           : rounds(std::integral_constant<int, 1>{});
+    // The rest of the row (all of it when unaligned): one distance per lane, waves interleaved.
+    for (int64_t b0 = full + static_cast<int64_t>(wave) * WAVE; b0 < len; b0 += W * WAVE) {
+        const int64_t j = b0 + lane;
+        const bool valid = j < len;
+        const float x = valid ? row[j] : INFINITY;
+        list.offer(x, static_cast<int32_t>(j), valid, K);
+    }
 }
 
 // Number of entries of the sorted list l[0..K) that precede e: strictly less when strict, else less-or-equal.

@@ -565,7 +565,7 @@ constexpr int wave_kernel_waves_per_simd() {
     return waves < 1 ? 1 : (waves > 4 ? 4 : waves);
 }
 
-// First slab whose granule range [slab_gran[s], slab_gran[s + 1]) contains `item` (binary search; inverted lists).
+// The last of `slabs` ascending starts at or below `item` (binary search; inverted lists).
 __device__ __forceinline__ int64_t slab_of(const int64_t* slab_gran, int64_t slabs, int64_t item) {
     int64_t lo = 0, hi = slabs - 1;
     while (lo < hi) {
@@ -576,10 +576,10 @@ __device__ __forceinline__ int64_t slab_of(const int64_t* slab_gran, int64_t sla
     return lo;
 }
 
-// IVF (one query per slab, QS = 1): the scan runs over inverted lists. Slab s is a list probed by query
-// a.slab_queries[s]; slabs are in query-major order, so a query's probed lists form one run of consecutive slabs,
+// IVF (one query per slab, QS = 1): the scan runs over inverted lists. Slab q * a.nprobe + p is the p-th list probed
+// by query q; slabs are in query-major order, so a query's probed lists form one run of consecutive slabs,
 // granules [a.query_gran[q], a.query_gran[q + 1]) of the balanced partition (a.query_gran[nq] = total). Slab s covers
-// granules [a.slab_gran[s], a.slab_gran[s + 1]) (possibly none), its list's padded tiles start at a.slab_tile[s] in
+// the granules from a.query_gran[q] + a.slab_gran[s] to the next slab's start (possibly none), its list's padded tiles start at a.slab_tile[s] in
 // the word-interleaved codes (the plan copies the list's first tile there, one dependent load fewer per slab than
 // looking it up by list), and the vector ids come from a.ids (-1 on padding). A block
 // gathers a query's tables and starts its lists once per run and writes them once, at the end of the run (or of
@@ -661,10 +661,17 @@ __global__ void __launch_bounds__(T)
 #pragma unroll
     for (int j = 0; j < kHi; ++j) hi[j] = 0x10000u;
 
-    // Inverted lists: the first slab of the block's range by binary search (the last slab starting at or before
-    // `start`, i.e. the non-empty one holding it); every later one is the next non-empty slab, so the search costs
-    // one chain of dependent loads per block, not one per slab.
-    int64_t next_slab = IVF && start < end ? slab_of(a.slab_gran, a.n_slabs, start) : 0;
+    // Inverted lists: the first slab of the block's range by binary search (the last query, then its last slab,
+    // starting at or before `start`, i.e. the non-empty one holding it); every later one is the next non-empty slab,
+    // so the search costs one chain of dependent loads per block, not one per slab.
+    int64_t ivf_q = 0;
+    int ivf_p = 0;
+    if constexpr (IVF) {
+        if (start < end) {
+            ivf_q = slab_of(a.query_gran, a.nq, start);
+            ivf_p = static_cast<int>(slab_of(a.slab_gran + ivf_q * a.nprobe, a.nprobe, start - a.query_gran[ivf_q]));
+        }
+    }
     // Bulk admission (device.hpp) for long lists; for inverted lists, whose partial lists cover a few probed lists
     // each, so that many of their candidates arrive while the list is filling; for one query per block; and where
     // the launch asks for it (BULK): a list admits about K ln(n / K) candidates over n, a third of the first 64
@@ -695,13 +702,21 @@ __global__ void __launch_bounds__(T)
     for (int64_t item = start; item < end;) {
         // The slab holding `item` and its granules [slab_first, slab_next) in the balanced partition.
         int64_t slab, slab_first, slab_next;
+        int32_t slab_query = 0;  // IVF
         if constexpr (IVF) {
             // Probes of no list or of an empty list are empty slabs: skipped (a non-empty slab holds `item`).
-            slab = next_slab;
-            while (a.slab_gran[slab + 1] == a.slab_gran[slab]) ++slab;
-            next_slab = slab + 1;
-            slab_first = a.slab_gran[slab];
-            slab_next = a.slab_gran[slab + 1];
+            for (;;) {
+                slab = ivf_q * a.nprobe + ivf_p;
+                const int64_t run = a.query_gran[ivf_q];
+                slab_first = run + a.slab_gran[slab];
+                slab_next = ivf_p + 1 < a.nprobe ? run + a.slab_gran[slab + 1] : a.query_gran[ivf_q + 1];
+                slab_query = static_cast<int32_t>(ivf_q);
+                if (++ivf_p == a.nprobe) {
+                    ivf_p = 0;
+                    ++ivf_q;
+                }
+                if (slab_next > slab_first) break;
+            }
         } else {
             slab = item / a.n_gran;
             slab_first = slab * a.n_gran;
@@ -717,7 +732,7 @@ __global__ void __launch_bounds__(T)
         bool live[QS];
         bool new_run = true;
         if constexpr (IVF) {
-            const int32_t qi = a.slab_queries[slab];
+            const int32_t qi = slab_query;
             new_run = qi != run_query;
             run_query = qi;
             qrow[0] = a.queries + static_cast<int64_t>(qi) * a.d;
@@ -774,6 +789,10 @@ __global__ void __launch_bounds__(T)
         // One granule step of this wave (g: the wave's granule, advanced at the end). bulk_step: candidates are
         // admitted in bulk whatever the list type.
         int64_t g = g_lo + wave;
+        // Inverted lists: granules go to waves by their number in the whole partition, so that a run of lists
+        // shorter than W granules keeps every wave busy (a list of four granules would otherwise always be the
+        // first four waves').
+        if constexpr (IVF) g = g_lo + ((wave - static_cast<int>(item)) & (W - 1));
         // Admission queue: merges list q's queued candidates into it. Lanes read slots that other lanes of the wave
         // wrote: the LDS serves one wave's accesses in order, and the wave barriers keep the compiler from moving
         // these reads above those writes, or the next appends above these reads.

@@ -9,6 +9,7 @@ namespace vk {
 
 WaveScanKernel ivf_kernel_m16(int segments);
 WaveScanKernel ivf_kernel_m32(int segments);
+WaveScanKernel ivf_kernel_m48(int segments);
 WaveScanKernel ivf_kernel_m64(int segments);
 WaveScanKernel ivf_kernel_mx(int segments);
 
@@ -16,6 +17,7 @@ WaveScanKernel ivf_kernel(int m, int segments) {
     switch (m) {
         case 16: return ivf_kernel_m16(segments);
         case 32: return ivf_kernel_m32(segments);
+        case 48: return ivf_kernel_m48(segments);
         case 64: return ivf_kernel_m64(segments);
         default: return ivf_kernel_mx(segments);
     }
@@ -25,7 +27,6 @@ namespace {
 
 constexpr int kMergeThreads = 256;
 constexpr int kPlanThreads = 256;
-constexpr int kScanThreads = 1024;
 
 __device__ __forceinline__ int64_t wave_inclusive_sum(int64_t v) {
     const int lane = __lane_id();
@@ -37,66 +38,71 @@ __device__ __forceinline__ int64_t wave_inclusive_sum(int64_t v) {
     return v;
 }
 
-// Plan, step 1 (one wave per query): slab q * nprobe + p is query q's p-th probed list; its granule count is the
-// list's padded tiles / 4 (0 for a probe of no list). slab_gran receives each slab's start within its query's run
-// and query_gran[q] the run's length.
-__global__ void __launch_bounds__(kPlanThreads) ivf_plan_runs_kernel(IvfPlanArgs a) {
-    const int lane = __lane_id();
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / WAVE);
-    const int64_t q = static_cast<int64_t>(blockIdx.x) * (kPlanThreads / WAVE) + wave;
-    if (q >= a.nq) return;  // wave-uniform
-    int64_t run = 0;
-    for (int base = 0; base < a.nprobe; base += WAVE) {
-        const int p = base + lane;
-        int64_t tile = 0;
-        int64_t gran = 0;
-        if (p < a.nprobe) {
-            const int32_t l = a.probes[q * a.nprobe + p].i;
-            if (l >= 0) {  // a query whose coarse distances are all NaN probes nothing
+// Probe selection and the slab plan, one block per query. Each wave streams its share of the query's coarse
+// distances into a wave list, the lists are merged by rank, and the nprobe nearest become slabs q * nprobe + p in
+// probe order: a slab's granule count is its list's padded tiles / 4 (0 for no list: a query whose coarse distances
+// are all NaN probes nothing), slab_gran receives its start within the query's run. The last block to finish (a
+// ticket, left at zero) turns the run lengths in query_gran[0..nq) into their exclusive prefix, query_gran[nq] = total.
+// One launch for what were four (row top-k, run lengths, prefix, absolute slab starts): a search of one query is a
+// chain of launches that each last a few microseconds.
+template <int S>
+__global__ void __launch_bounds__(kPlanThreads) ivf_plan_kernel(IvfPlanArgs a) {
+    constexpr int W = kPlanThreads / WAVE;
+    __shared__ Pair buf[(W + 1) * WAVE * S];
+    __shared__ int64_t wave_sums[W];
+    __shared__ bool last_block;
+    const int tid = threadIdx.x, lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int64_t q = a.first + blockIdx.x;
+    WaveList<S, true> list;
+    list.init();
+    stream_row<S, W>(list, a.dists + static_cast<int64_t>(blockIdx.x) * a.nlist, a.nlist, a.K, wave, lane);
+    Pair* const merged = buf + W * a.K;
+    list.store(buf + wave * a.K, a.K);
+    __syncthreads();
+    merge_lists(buf, W, a.K, merged, tid, kPlanThreads);
+    __syncthreads();
+    if (wave == 0) {
+        int64_t run = 0;
+        for (int base = 0; base < a.nprobe; base += WAVE) {
+            const int p = base + lane;
+            int64_t tile = 0, gran = 0;
+            if (p < a.nprobe && merged[p].i != kEmptyId) {
+                const int32_t l = merged[p].i;
                 tile = a.list_tile[l];
                 gran = (a.list_tile[l + 1] - tile) / 4;
             }
+            const int64_t incl = wave_inclusive_sum(gran);
+            if (p < a.nprobe) {
+                const int64_t s = q * a.nprobe + p;
+                a.slab_tile[s] = tile;
+                a.slab_gran[s] = run + incl - gran;
+            }
+            run += __shfl(incl, WAVE - 1);
         }
-        const int64_t incl = wave_inclusive_sum(gran);
-        if (p < a.nprobe) {
-            const int64_t s = q * a.nprobe + p;
-            a.slab_tile[s] = tile;
-            a.slab_queries[s] = static_cast<int32_t>(q);
-            a.slab_gran[s] = run + incl - gran;
+        if (lane == 0) {
+            a.query_gran[q] = run;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            last_block = atomicInc(a.ticket, static_cast<unsigned>(a.nq - 1)) == static_cast<unsigned>(a.nq - 1);
         }
-        run += __shfl(incl, WAVE - 1);
     }
-    if (lane == 0) a.query_gran[q] = run;
-}
-
-// Plan, step 2 (one block): query_gran[0..nq) from run lengths to their exclusive prefix, query_gran[nq] = total.
-__global__ void __launch_bounds__(kScanThreads) ivf_plan_scan_kernel(IvfPlanArgs a) {
-    __shared__ int64_t wave_sums[kScanThreads / WAVE];
-    const int tid = threadIdx.x, lane = __lane_id(), wave = tid / WAVE;
-    const int64_t per = (a.nq + kScanThreads - 1) / kScanThreads;
+    __syncthreads();
+    if (!last_block) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    const int64_t per = (a.nq + kPlanThreads - 1) / kPlanThreads;
     const int64_t lo = min<int64_t>(a.nq, tid * per), hi = min<int64_t>(a.nq, lo + per);
     int64_t sum = 0;
     for (int64_t i = lo; i < hi; ++i) sum += a.query_gran[i];
     const int64_t incl = wave_inclusive_sum(sum);
     if (lane == WAVE - 1) wave_sums[wave] = incl;
     __syncthreads();
-    int64_t before = 0;
-    for (int w = 0; w < wave; ++w) before += wave_sums[w];
-    int64_t run = before + incl - sum;
+    int64_t run = incl - sum;
+    for (int w = 0; w < wave; ++w) run += wave_sums[w];
     for (int64_t i = lo; i < hi; ++i) {
         const int64_t len = a.query_gran[i];
         a.query_gran[i] = run;
         run += len;
     }
-    if (tid == kScanThreads - 1) a.query_gran[a.nq] = run;
-}
-
-// Plan, step 3 (one thread per slab): slab starts from run-relative to absolute; slab_gran[n_slabs] = total.
-__global__ void __launch_bounds__(kPlanThreads) ivf_plan_offsets_kernel(IvfPlanArgs a) {
-    const int64_t s = static_cast<int64_t>(blockIdx.x) * kPlanThreads + threadIdx.x;
-    const int64_t slabs = a.nq * a.nprobe;
-    if (s < slabs) a.slab_gran[s] += a.query_gran[s / a.nprobe];
-    if (s == slabs) a.slab_gran[s] = a.query_gran[a.nq];
+    if (tid == kPlanThreads - 1) a.query_gran[a.nq] = run;
 }
 
 // One wave per query streams its partial lists through a wave list (device.hpp: whole lists when long, else
@@ -129,15 +135,12 @@ __global__ void __launch_bounds__(kMergeThreads) ivf_merge_kernel(IvfMergeArgs a
 
 }  // namespace
 
-hipError_t launch_ivf_plan(const IvfPlanArgs& a, hipStream_t stream) {
-    if (a.nq <= 0 || a.nprobe <= 0) return hipErrorInvalidValue;
-    const int waves = kPlanThreads / WAVE;
-    hipLaunchKernelGGL(ivf_plan_runs_kernel, dim3(static_cast<unsigned>((a.nq + waves - 1) / waves)),
-                       dim3(kPlanThreads), 0, stream, a);
-    hipLaunchKernelGGL(ivf_plan_scan_kernel, dim3(1), dim3(kScanThreads), 0, stream, a);
-    const int64_t slabs = a.nq * a.nprobe + 1;
-    hipLaunchKernelGGL(ivf_plan_offsets_kernel, dim3(static_cast<unsigned>((slabs + kPlanThreads - 1) / kPlanThreads)),
-                       dim3(kPlanThreads), 0, stream, a);
+hipError_t launch_ivf_plan(const IvfPlanArgs& a, int rows, hipStream_t stream) {
+    if (a.nq <= 0 || a.nprobe <= 0 || rows <= 0) return hipErrorInvalidValue;
+    const dim3 grid(static_cast<unsigned>(rows));
+    if (a.K <= WAVE) hipLaunchKernelGGL(ivf_plan_kernel<1>, grid, dim3(kPlanThreads), 0, stream, a);
+    else if (a.K <= 2 * WAVE) hipLaunchKernelGGL(ivf_plan_kernel<2>, grid, dim3(kPlanThreads), 0, stream, a);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

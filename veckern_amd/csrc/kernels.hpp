@@ -65,10 +65,9 @@ struct WaveScanArgs {
     Pair* out;               // [nq][k]; empty slots become {+inf, -1}
     // Inverted lists (IVF instances only, one query per slab, the plan of launch_ivf_plan); `n_gran`, `total` and
     // `max_slots` are then unused (the total is query_gran[nq]).
-    int64_t n_slabs;
-    const int64_t* slab_gran;      // [n_slabs + 1] granule prefix of the slabs
-    const int64_t* slab_tile;      // [n_slabs] first tile in `codes` / `ids` of the list each slab scans
-    const int32_t* slab_queries;   // [n_slabs] query of each slab; a query's slabs are consecutive
+    int nprobe;                    // slabs per query; slab q * nprobe + p is query q's p-th probed list
+    const int64_t* slab_gran;      // [nq * nprobe] granule start of the slabs within their query's run
+    const int64_t* slab_tile;      // [nq * nprobe] first tile in `codes` / `ids` of the list each slab scans
     const int64_t* query_gran;     // [nq + 1] granule prefix of the queries' runs of slabs
     const int64_t* list_tile;      // [lists + 1] first tile of each list in `codes` / `ids`
     const int32_t* ids;            // [tiles * 64] vector id of each padded position, -1 for padding
@@ -90,26 +89,37 @@ WaveScanKernel fused_wave_kernel(int qg, int ng, int ilp, int m, int segments, b
 // The inverted-list scan (ivf_m*.hip): fp32 tables, one query per slab, four tiles per wave step.
 WaveScanKernel ivf_kernel(int m, int segments);
 
-// ---- IVF plan (ivf.hip): from the probes (nq x nprobe, id -1 = no list), slab q * nprobe + p = query q's p-th
-// probed list: slab_tile (the list's first tile) / slab_queries [nq * nprobe], slab_gran [nq * nprobe + 1] (granule
-// starts; a probe of no
-// list or of an empty list is an empty slab), query_gran [nq + 1] (the granule start of each query's run; the last
-// entry is the total).
+// ---- IVF plan (ivf.hip), device only, for query-major slabs: from the coarse distances of queries first ..
+// first + rows - 1 (dists [rows][nlist]), slab q * nprobe + p is query q's p-th nearest list: slab_tile (the list's
+// first tile) and slab_gran (its granule start within the query's run; a probe of no list or of an empty list is an
+// empty slab), both [nq * nprobe]; query_gran [nq + 1] (the granule start of each query's run; the last entry is the
+// total) is complete once every row has been planned. ticket: zero between searches.
 struct IvfPlanArgs {
-    const Pair* probes;
+    const float* dists;
+    int64_t nlist;
+    int64_t first;
+    int K;  // list length (dispatched nprobe)
     int nprobe;
     int64_t nq;
     const int64_t* list_tile;
     int64_t* slab_tile;
-    int32_t* slab_queries;
     int64_t* slab_gran;
     int64_t* query_gran;
+    unsigned* ticket;
 };
-hipError_t launch_ivf_plan(const IvfPlanArgs& a, hipStream_t stream);
+hipError_t launch_ivf_plan(const IvfPlanArgs& a, int rows, hipStream_t stream);
 
-// ---- IVF probe (probe.hip): out[q][l] = exact squared L2 distance of query q to coarse centroid l (nq x nlist)
+// ---- IVF probe (probe.hip): out[q][l] = exact squared L2 distance of query q to coarse centroid l (nq x nlist). With
+// lut.queries set, the same launch also writes the tables lut.out[q][s][c] of lut.nq queries (as launch_lut, qg = 1).
+struct ProbeLut {
+    const float* queries;
+    const float* centroids;
+    int m;
+    int nq;
+    float* out;
+};
 hipError_t launch_coarse_distances(const float* queries, int64_t nq, const float* coarse, int64_t nlist, int d,
-                                   float* out, hipStream_t stream);
+                                   float* out, const ProbeLut& lut, hipStream_t stream);
 // list_ids[i] = the nearest coarse centroid of vector i by (exact squared L2 distance, centroid index)
 hipError_t launch_coarse_assign(const float* x, int64_t n, const float* coarse, int64_t nlist, int d,
                                 int32_t* list_ids, hipStream_t stream);

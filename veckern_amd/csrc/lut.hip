@@ -6,6 +6,7 @@
 // plain [q][s][c] layout (QG = 1) has its own kernel below. The query sub-vector is
 // block-uniform, so it is read through scalar loads; the centroid row is read once and reused for all QG queries.
 #include "kernels.hpp"
+#include "lut_rows.hpp"
 
 namespace vk {
 
@@ -36,45 +37,12 @@ __global__ void __launch_bounds__(KSUB)
     for (int qq = 0; qq < QG; ++qq) dst[qq] = out[qq];
 }
 
-// The plain [q][s][c] layout (QG = 1), G queries per block: thread c reads centroid c of sub-space s once (DSUB
-// known at compile time: one or two 16-byte loads) and produces its entry for each of the G queries, each store
-// coalesced over c. A block per (s, query) would reread the centroid row G times and leave each thread one entry.
-constexpr int kLutQueries = 8;
-
+// The plain [q][s][c] layout (QG = 1).
 template <int DSUB>
 __global__ void __launch_bounds__(KSUB)
     lut_rows_kernel(const float* __restrict__ queries, const float* __restrict__ centroids, int d, int m, int dsub_rt,
                     int nq, float* __restrict__ lut) {
-#pragma clang fp contract(off)
-    const int dsub = DSUB ? DSUB : dsub_rt;
-    const int s = blockIdx.x, c = threadIdx.x;
-    const int q0 = blockIdx.y * kLutQueries;
-    const float* cent = centroids + (static_cast<size_t>(s) * KSUB + c) * dsub;
-    float cv[DSUB ? DSUB : 1];
-    if constexpr (DSUB > 0) {
-#pragma unroll
-        for (int j = 0; j < DSUB; ++j) cv[j] = cent[j];
-    }
-#pragma unroll
-    for (int qq = 0; qq < kLutQueries; ++qq) {
-        const int q = q0 + qq;
-        if (q >= nq) break;  // block-uniform
-        const float* x = queries + static_cast<size_t>(q) * d + static_cast<size_t>(s) * dsub;
-        float acc = 0.f;
-        if constexpr (DSUB > 0) {
-#pragma unroll
-            for (int j = 0; j < DSUB; ++j) {
-                const float diff = x[j] - cv[j];
-                acc += diff * diff;
-            }
-        } else {
-            for (int j = 0; j < dsub; ++j) {
-                const float diff = x[j] - cent[j];
-                acc += diff * diff;
-            }
-        }
-        lut[(static_cast<size_t>(q) * m + s) * KSUB + c] = acc;
-    }
+    lut_rows<DSUB>(queries, centroids, d, m, dsub_rt, nq, lut, blockIdx.x, blockIdx.y * kLutQueries, threadIdx.x);
 }
 
 hipError_t launch_lut(const float* queries, const float* centroids, int d, int m, int nq, int qg, int groups,

@@ -13,6 +13,7 @@
 #include <climits>
 
 #include "kernels.hpp"
+#include "lut_rows.hpp"
 
 namespace vk {
 
@@ -97,13 +98,24 @@ __device__ __forceinline__ void tile_sums(const float* __restrict__ x, int64_t n
 // stage 0.048 -> 0.044 ms; 1 x 4 per thread gave 0.046).
 constexpr int kProbeRQ = 2, kProbeCJ = 2;
 
+// The first lut_blocks blocks build the search's tables instead of a tile: neither needs the other, and a launch of
+// their own cost a search of one query as much as the work.
+template <int DSUB>
 __global__ void __launch_bounds__(kThreads) coarse_distance_kernel(const float* __restrict__ queries, int64_t nq,
                                                                   const float* __restrict__ coarse, int64_t nlist,
-                                                                  int d, float* __restrict__ out) {
+                                                                  int d, float* __restrict__ out, ProbeLut lut,
+                                                                  int lut_blocks, int tiles_l) {
+    static_assert(kThreads == KSUB, "a table block has a thread per centroid");
     __shared__ __align__(16) Tile<kProbeRQ, kProbeCJ> sm;
     const int tid = threadIdx.x, ty = tid / 16, tx = tid % 16;
-    const int64_t q0 = static_cast<int64_t>(blockIdx.y) * Tile<kProbeRQ, kProbeCJ>::kQ;
-    const int64_t l0 = static_cast<int64_t>(blockIdx.x) * Tile<kProbeRQ, kProbeCJ>::kL;
+    const int block = static_cast<int>(blockIdx.x);
+    if (block < lut_blocks) {
+        lut_rows<DSUB>(lut.queries, lut.centroids, d, lut.m, d / lut.m, lut.nq, lut.out, block % lut.m,
+                       block / lut.m * kLutQueries, tid);
+        return;
+    }
+    const int64_t q0 = static_cast<int64_t>((block - lut_blocks) / tiles_l) * Tile<kProbeRQ, kProbeCJ>::kQ;
+    const int64_t l0 = static_cast<int64_t>((block - lut_blocks) % tiles_l) * Tile<kProbeRQ, kProbeCJ>::kL;
     float acc[kProbeRQ][kProbeCJ];
     tile_sums(queries, nq, coarse, nlist, d, q0, l0, sm, acc);
 #pragma unroll
@@ -167,11 +179,18 @@ __global__ void __launch_bounds__(kThreads) coarse_assign_kernel(const float* __
 }  // namespace
 
 hipError_t launch_coarse_distances(const float* queries, int64_t nq, const float* coarse, int64_t nlist, int d,
-                                   float* out, hipStream_t stream) {
+                                   float* out, const ProbeLut& lut, hipStream_t stream) {
     constexpr int kQ = Tile<kProbeRQ, kProbeCJ>::kQ, kL = Tile<kProbeRQ, kProbeCJ>::kL;
-    if (nq <= 0 || nlist <= 0 || d <= 0 || (nq + kQ - 1) / kQ > 65535) return hipErrorInvalidValue;
-    const dim3 grid(static_cast<unsigned>((nlist + kL - 1) / kL), static_cast<unsigned>((nq + kQ - 1) / kQ));
-    hipLaunchKernelGGL(coarse_distance_kernel, grid, dim3(kThreads), 0, stream, queries, nq, coarse, nlist, d, out);
+    if (nq <= 0 || nlist <= 0 || d <= 0) return hipErrorInvalidValue;
+    const int64_t tiles_l = (nlist + kL - 1) / kL, tiles = tiles_l * ((nq + kQ - 1) / kQ);
+    const int64_t lut_blocks =
+        lut.queries ? static_cast<int64_t>(lut.m) * ((lut.nq + kLutQueries - 1) / kLutQueries) : 0;
+    if (tiles + lut_blocks >= int64_t{1} << 24) return hipErrorInvalidValue;  // 2^32 threads in one dimension
+    const int dsub = lut.queries ? d / lut.m : 0;
+    auto kernel = dsub == 8 ? coarse_distance_kernel<8> : dsub == 4 ? coarse_distance_kernel<4>
+                                                        : dsub == 2 ? coarse_distance_kernel<2> : coarse_distance_kernel<0>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles + lut_blocks)), dim3(kThreads), 0, stream, queries, nq,
+                       coarse, nlist, d, out, lut, static_cast<int>(lut_blocks), static_cast<int>(tiles_l));
     return hipGetLastError();
 }
 
