@@ -1,0 +1,8 @@
+// Instances of the fused wave-list scan that abandon tiles, fp16 tables, m = 16.
+#include "fused_wave.inl"
+
+namespace vk {
+WaveScanKernel abandon_kernel_h16(int q, int segments, int threads) {
+    return select_abandon_kernel<16, true>(q, segments, threads);
+}
+}  // namespace vk

@@ -1,0 +1,8 @@
+// Instances of the fused wave-list scan that abandon tiles, fp16 tables, m = 64.
+#include "fused_wave.inl"
+
+namespace vk {
+WaveScanKernel abandon_kernel_h64(int q, int segments, int threads) {
+    return select_abandon_kernel<64, true>(q, segments, threads);
+}
+}  // namespace vk

@@ -1,0 +1,8 @@
+// Instances of the fused wave-list scan that abandon tiles, fp32 tables, m = 64.
+#include "fused_wave.inl"
+
+namespace vk {
+WaveScanKernel abandon_kernel_m64(int q, int segments, int threads) {
+    return select_abandon_kernel<64, false>(q, segments, threads);
+}
+}  // namespace vk

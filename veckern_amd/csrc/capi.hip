@@ -35,6 +35,25 @@ WaveScanKernel fused_wave_kernel_h48(int qg, int ng, int ilp, int segments, bool
 WaveScanKernel fused_wave_kernel_h64(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_hx(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 
+WaveScanKernel abandon_kernel_m16(int q, int segments, int threads);
+WaveScanKernel abandon_kernel_m32(int q, int segments, int threads);
+WaveScanKernel abandon_kernel_m48(int q, int segments, int threads);
+WaveScanKernel abandon_kernel_m64(int q, int segments, int threads);
+WaveScanKernel abandon_kernel_h16(int q, int segments, int threads);
+WaveScanKernel abandon_kernel_h32(int q, int segments, int threads);
+WaveScanKernel abandon_kernel_h48(int q, int segments, int threads);
+WaveScanKernel abandon_kernel_h64(int q, int segments, int threads);
+
+WaveScanKernel abandon_kernel(int q, int m, int segments, bool f16, int threads) {
+    switch (m) {
+        case 16: return f16 ? abandon_kernel_h16(q, segments, threads) : abandon_kernel_m16(q, segments, threads);
+        case 32: return f16 ? abandon_kernel_h32(q, segments, threads) : abandon_kernel_m32(q, segments, threads);
+        case 48: return f16 ? abandon_kernel_h48(q, segments, threads) : abandon_kernel_m48(q, segments, threads);
+        case 64: return f16 ? abandon_kernel_h64(q, segments, threads) : abandon_kernel_m64(q, segments, threads);
+        default: return WaveScanKernel{};
+    }
+}
+
 WaveScanKernel fused_wave_kernel(int qg, int ng, int ilp, int m, int segments, bool f16, bool bulk, int threads) {
     if (f16) {
         switch (m) {
@@ -259,6 +278,8 @@ struct vk_searcher {
     hipStream_t stream = nullptr;
     DeviceBuffer<float> centroids, queries, lut, dists;
     DeviceBuffer<uint8_t> codes, codes_il;
+    DeviceBuffer<uint4> heads;             // the first codes of the sorted layout (abandon_tiles)
+    bool abandon_tiles = false;            // the codes repeat within tiles: scans with abandoned tiles
     DeviceBuffer<uint4> codes_v, codes_s;  // words in vector order (v6, v7) and in sorted slot order (v8, v9)
     DeviceBuffer<uint32_t> slot_ids;        // the sorted slot order: the vector id of each slot (m % 16 == 0 only)
     DeviceBuffer<uint8_t> table_rows;       // [m][256]: the LDS table row of each code value in the sorted layout
@@ -304,9 +325,31 @@ struct vk_searcher {
             codes_s.ensure(static_cast<size_t>(n_pad) * (m / 16));
             VK_HIP(vk::launch_build_sorted_words(codes.get(), n, static_cast<int>(m), n_pad, slot_ids.get(),
                                                  table_rows.get(), codes_s.get(), stream));
+            choose_abandon();
             have_s = built = true;
         }
         if (built) VK_HIP(hipStreamSynchronize(stream));  // a layout kernel's failure surfaces here, not mid-search
+    }
+
+    // Whether the v8/v9 scans abandon tiles: a tile is dropped when all of its 64 vectors are beyond every bound, which
+    // happens early where the vectors of a tile are close to each other and hardly ever where they are not. Measured as
+    // how far apart the vectors of neighbouring slots are, against vectors half the database apart, in sampled tiles.
+    void choose_abandon() {
+        const int64_t tiles = static_cast<int64_t>(n) / vk::WAVE;
+        if (m > 64 || tiles < 2) return;
+        DeviceBuffer<double> spread;
+        spread.ensure(2);
+        VK_HIP(vk::launch_zero_words(reinterpret_cast<unsigned*>(spread.get()), 4, stream));
+        VK_HIP(vk::launch_tile_spread(codes.get(), slot_ids.get(), centroids.get(), static_cast<int>(m),
+                                      static_cast<int>(d / m), tiles, (tiles + 1023) / 1024, spread.get(), stream));
+        double sums[2] = {0.0, 0.0};
+        VK_HIP(hipMemcpyAsync(sums, spread.get(), sizeof sums, hipMemcpyDeviceToHost, stream));
+        VK_HIP(hipStreamSynchronize(stream));
+        abandon_tiles = vk::plan::abandon_pays(sums[0], sums[1]);
+        if (!abandon_tiles) return;
+        const int words = vk::abandon_head_words(static_cast<int>(m));
+        heads.ensure(static_cast<size_t>(n_pad / 256) * words * vk::WAVE);
+        VK_HIP(vk::launch_build_heads(codes_s.get(), static_cast<int>(m), n_pad, words, heads.get(), stream));
     }
 
     // The slot order and table rows of the fused scans' layout (slot_order.hpp), for table reads of `lanes` lanes
@@ -396,7 +439,14 @@ struct vk_searcher {
         // fp32: 8 queries are two groups of 4 (16-byte reads); fp16: up to 8 queries in one group.
         const int qg = (!f16 && w.q == 8) ? 4 : w.q, ng = (!f16 && w.q == 8) ? 2 : 1;
         w.ilp = tuning.vectors_per_step;
-        w.kern = vk::fused_wave_kernel(qg, ng, w.ilp, static_cast<int>(m), segments, f16);
+        bool abandon = false;
+        if (abandon_tiles && w.ilp == 4 && ng == 1) {
+            if (tuning.scan_threads != 512)
+                w.kern = vk::abandon_kernel(w.q, static_cast<int>(m), segments, f16, 1024);
+            if (!w.kern.fn) w.kern = vk::abandon_kernel(w.q, static_cast<int>(m), segments, f16, 512);
+            abandon = w.kern.fn != nullptr;
+        }
+        if (!abandon) w.kern = vk::fused_wave_kernel(qg, ng, w.ilp, static_cast<int>(m), segments, f16);
         if (!w.kern.fn) fail(VK_ERR_LOGIC, "no fused-warp kernel built for this (Q, ILP, m, K)");
         const size_t tables = static_cast<size_t>(w.q) * m * vk::KSUB * entry_bytes;
         require(tables <= info.max_smem_per_block, "LUT does not fit in LDS");
@@ -415,7 +465,7 @@ struct vk_searcher {
         // bulk-scan bound; and not crossing slab boundaries where 512-thread blocks would not): one block per CU,
         // whose 16 waves share one granule counter, instead of two 512-thread blocks that the CU does not balance
         // or one of 8 waves. scan_threads = 512 or 1024 pins the block size.
-        if (tuning.scan_threads != 512) {
+        if (!abandon && tuning.scan_threads != 512) {
             const vk::WaveScanKernel wide =
                 vk::fused_wave_kernel(qg, ng, w.ilp, static_cast<int>(m), segments, f16, false, 1024);
             if (wide.fn) {
@@ -433,7 +483,7 @@ struct vk_searcher {
         }
         // Few vectors per block: the instance that admits candidates in bulk, if it has the same residency (the
         // partition above was planned with it).
-        if (!f16 && segments == 1 && w.q > 1 && vk::plan::bulk_scan(w.part, w.ilp)) {
+        if (!abandon && !f16 && segments == 1 && w.q > 1 && vk::plan::bulk_scan(w.part, w.ilp)) {
             const vk::WaveScanKernel bulk = vk::fused_wave_kernel(qg, ng, w.ilp, static_cast<int>(m), segments, f16,
                                                                   true, w.kern.threads);
             int bulk_per_cu = 0;
@@ -455,7 +505,7 @@ struct vk_searcher {
     // One launch of a planned wave-list scan over this batch's b device queries d_q into d_out (b x kk). part and
     // counters: scratch of w.part_pairs pairs and w.part.slabs zeroed counters (the kernel leaves them at zero).
     void launch_wave(const WavePlan& w, const float* d_q, size_t b, size_t kk, Pair* d_out, Pair* part_buf,
-                     unsigned* counter_buf) {
+                     unsigned* counter_buf, unsigned* bound_buf) {
         last = vk_launch_shape{};
         last.threads = w.kern.threads;
         last.blocks_x = static_cast<int>(w.part.grid);
@@ -485,6 +535,8 @@ struct vk_searcher {
         a.lists_per_block = w.lists_per_block;
         a.part = part_buf;
         a.counters = counter_buf;
+        a.bounds = bound_buf;
+        a.heads = heads.get();
         a.out = d_out;
         VK_HIP(w.kern.launch(a, static_cast<int>(w.part.grid), w.smem, stream));
     }
@@ -494,13 +546,16 @@ struct vk_searcher {
     void run_wave(const float* d_q, size_t b, size_t kk, bool f16, Pair* d_out, vk_timings* t, StageClock& clock) {
         const WavePlan w = plan_wave(b, kk, f16);
         part.ensure(w.part_pairs);
-        ensure_counters(static_cast<size_t>(w.part.slabs));
+        const size_t slabs = static_cast<size_t>(w.part.slabs);
+        ensure_counters(slabs + slabs * static_cast<size_t>(w.q));
         counters_dirty = true;  // cleared once the stream completes the launch without error
-        clock.time(&t->scan_ms, [&] { launch_wave(w, d_q, b, kk, d_out, part.get(), counters.get()); });
+        clock.time(&t->scan_ms, [&] {
+            launch_wave(w, d_q, b, kk, d_out, part.get(), counters.get(), counters.get() + slabs);
+        });
     }
 
-    // Per-slab completion counters of the wave-list scan. The kernel leaves them at zero; they are zeroed here
-    // when allocated or grown, and again if a previous launch may have stopped part way (an error was raised
+    // Per-slab completion counters and per-query shared bounds of the wave-list scan (`slabs`: words of both). The
+    // kernel leaves them at zero; they are zeroed here when allocated or grown, and again if a previous launch may have stopped part way (an error was raised
     // between the launch and the stream's completion).
     void ensure_counters(size_t slabs) {
         if (slabs > counters_zeroed || counters_dirty) {
@@ -730,8 +785,13 @@ struct vk_searcher {
         dev.counters_clean = false;  // until the stream has completed every launch below
         for (size_t q0 = 0; q0 < nq; q0 += batch) {
             const size_t b = std::min(batch, nq - q0);
-            launch_wave(plan_wave(b, kk, f16), d_q + q0 * d, b, kk, reinterpret_cast<Pair*>(d_out + q0 * kk),
-                        part_buf, counter_buf);
+            const WavePlan w = plan_wave(b, kk, f16);
+            // The shared bounds sit behind the counters where both fit; without them the slab's blocks scan with
+            // their own bounds only (same results).
+            const size_t slabs = static_cast<size_t>(w.part.slabs);
+            const bool fit = (slabs + slabs * static_cast<size_t>(w.q)) * sizeof(unsigned) <= kNoAllocCounterBytes;
+            launch_wave(w, d_q + q0 * d, b, kk, reinterpret_cast<Pair*>(d_out + q0 * kk), part_buf, counter_buf,
+                        fit ? counter_buf + slabs : nullptr);
         }
         VK_HIP(hipStreamSynchronize(stream));
         dev.counters_clean = true;

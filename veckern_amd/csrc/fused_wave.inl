@@ -584,7 +584,7 @@ __device__ __forceinline__ int64_t slab_of(const int64_t* slab_gran, int64_t sla
 // looking it up by list), and the vector ids come from a.ids (-1 on padding). A block
 // gathers a query's tables and starts its lists once per run and writes them once, at the end of the run (or of
 // its range); a separate merge kernel combines the partial lists of each query.
-template <int QG, int NG, int U, int M, int S, int T, bool F16, bool IVF, bool BULK>
+template <int QG, int NG, int U, int M, int S, int T, bool F16, bool IVF, bool BULK, bool ABANDON = false>
 __global__ void __launch_bounds__(T)
     __attribute__((amdgpu_waves_per_eu(wave_kernel_waves_per_simd<QG, NG, M, T, F16>())))
     fused_wave_kernel_t(WaveScanArgs a) {
@@ -605,6 +605,29 @@ __global__ void __launch_bounds__(T)
     // SIMD to finish the block, too few to keep the LDS pipe busy.
     __shared__ unsigned next_gran;
     __shared__ unsigned qmax[QS];  // fp16 tables: per-query maximum entry of the current slab (raw bits)
+    // Abandoned tiles (ABANDON; m fixed, four tiles per step, fp32 tables in one group or fp16): a tile's sums are
+    // compared with the admission bounds after its first sub-spaces, and the tile is dropped when no lane can be admitted
+    // by any query. Entries are sums of squares, so a running sum never falls (rounding to nearest is monotone): a
+    // partial sum beyond the bound means a distance beyond it, and a NaN stays a NaN, which no list admits. The bound
+    // of a query is the smallest of
+    //  - the K-th best distance of any wave's list in the block, and for K > 64 the second smallest of the waves'
+    //    ceil(K/2)-th best (two waves then hold K candidates at or below it), in block_bound;
+    //  - where several blocks share a slab, the bounds of its other blocks (a.bounds).
+    // K real candidates lie at or below it, so nothing beyond it reaches the merged top K; ties at it are kept.
+    // In the sorted slot order a tile's vectors are alike, so they fail together: on the 1M-vector Gaussian mixture 98 %
+    // of the tiles fail for all four queries after 6 of 16 sub-spaces (65 % after 4), 90 % after 8 of 32.
+    // The first kHeadBytes codes of every vector are read from an array of their own (a.heads): the scan reads half of
+    // the code bytes at m = 16 and a quarter at m = 32 .. 64, the rest and the ids only for tiles that are left.
+    constexpr bool kPrune = ABANDON;
+    static_assert(!ABANDON || (M > 0 && M <= 64 && U == 4 && NG == 1 && !IVF && !BULK), "instances that abandon tiles");
+    constexpr int kHeadWords = M <= 32 ? 2 : M / 16;  // dwords per vector
+    constexpr int kHeadBytes = 4 * kHeadWords;
+    // The first check: a quarter of the sub-spaces; at m = 16 a quarter lets a third of the tiles of four queries
+    // through, two more sub-spaces (10 VALU per tile) stop nearly all of those.
+    constexpr int kCheck = M == 16 && QS >= 4 ? 6 : M / 4;
+    __shared__ unsigned block_bound[QS];  // raw bits of a distance >= 0 or +inf: unsigned order is float order
+    constexpr bool kHalfRank = kPrune && S > 1;
+    __shared__ int half_rank[kHalfRank ? QS : 1][W];  // raw bits of the waves' ceil(K/2)-th best
     // Long lists (K > 64), and the bulk instances (few vectors per block): per (query, wave), the distance of the
     // wave list's entry ceil(K/W) - 1 for the current slab (raw bits of a distance >= 0, so unsigned order is float
     // order; +inf until the list holds that many). If every wave holds ceil(K/W) entries at or below T, the block
@@ -614,12 +637,12 @@ __global__ void __launch_bounds__(T)
     // (measured with the lane-parallel form below: 1M x nq=1000 +0.5 %, 10M +0.8 %, fp16 tables at 8 queries
     // +4.7 %); with few vectors per block, where a larger share of the candidates enters fresh lists, it pays
     // (100k x nq=100: -2 %).
-    constexpr bool kShareBound = S > 1 || (BULK && !IVF);
+    constexpr bool kShareBound = !kPrune && (S > 1 || (BULK && !IVF));
     // When every (query, wave) slot fits in one wave, a step reads all of them with one LDS read (lane l: slot l)
     // and takes each query's maximum over its W lanes by DPP exchanges; a wave publishes its QS values with one
     // LDS write (lane q: query q), always (they only fall).
     constexpr bool kLaneBound = kShareBound && QS * W <= WAVE && (W == 2 || W == 4 || W == 8 || W == 16);
-    __shared__ __align__(16) unsigned rank_bound[QS][W];
+    __shared__ __align__(16) unsigned rank_bound[kShareBound ? QS : 1][W];
     // Admission queue of the wave lists (fp32 tables, static LDS): candidates that pass a list's filter a few at a
     // time are appended to a run of kQueueCap LDS slots of their (query, wave) instead of being inserted one by one
     // (~22 VALU instructions each into a one-register list, ~32 into a two-register one). A full run and the end of
@@ -691,7 +714,7 @@ __global__ void __launch_bounds__(T)
     // few waves per CU leave that latency open otherwise. The multi-query instances read codes mostly from L2 and
     // need the registers for their accumulators (four queries, sorted codes, slab-aligned blocks: 1M x nq=1000
     // +4.5 % with the prefetch, 10M +3.6 %).
-    constexpr bool kPrefetch = !IVF && QS == 1 && M == 16;
+    constexpr bool kPrefetch = !IVF && QS == 1 && M == 16 && !kPrune;
     // Several code words per tile, or two tables, in a 1024-thread block (128 VGPRs): loading all U tiles' words at
     // the step's start spilled the later tiles' words to scratch in every step (m=32, k=100: 1 GB of scratch writes
     // per search), so each tile's words are loaded as the tile before it starts.
@@ -771,7 +794,10 @@ __global__ void __launch_bounds__(T)
             else build_tables<QG, NG, M, W, F16>(a, qrow, tables, qmax, wave, lane);
             if constexpr (kShareBound)
                 for (int t = tid; t < QS * W; t += T) (&rank_bound[0][0])[t] = 0x7f800000u;  // +inf
-            if (!IVF && tid == 0) next_gran = W;
+            if (!IVF && tid == 0) next_gran = kPrune ? 2 * W : W;
+            if (kPrune && tid < QS) block_bound[tid] = 0x7f800000u;  // +inf
+            if constexpr (kHalfRank)
+                for (int t = tid; t < QS * W; t += T) (&half_rank[0][0])[t] = 0x7f800000;
             __syncthreads();
 
             // A padded query slot (past nq in the last slab) gets the threshold -inf: no distance passes it, so
@@ -793,6 +819,11 @@ __global__ void __launch_bounds__(T)
         // shorter than W granules keeps every wave busy (a list of four granules would otherwise always be the
         // first four waves').
         if constexpr (IVF) g = g_lo + ((wave - static_cast<int>(item)) & (W - 1));
+        int64_t g_ahead = g + W;  // kPrune: the granule after g
+        // The blocks of this slab: first and count (exhaustive search).
+        const int64_t slab_lo = IVF ? 0 : first_block_of(slab_first, grid, total);
+        const int slab_blocks = IVF ? 1 : static_cast<int>(first_block_of(slab_next - 1, grid, total) - slab_lo + 1);
+        unsigned* const shared_bounds = kPrune && !IVF && slab_blocks > 1 && a.bounds ? a.bounds + slab * QS : nullptr;
         // Admission queue: merges list q's queued candidates into it. Lanes read slots that other lanes of the wave
         // wrote: the LDS serves one wave's accesses in order, and the wave barriers keep the compiler from moving
         // these reads above those writes, or the next appends above these reads.
@@ -1052,15 +1083,311 @@ __global__ void __launch_bounds__(T)
             if constexpr (IVF) g += W;
             else g = g_lo + static_cast<int64_t>(__builtin_amdgcn_readfirstlane(grab));
         };
+        // Lane l % W holds wave l % W's value: the second smallest of the W (equal values count each).
+        auto second_smallest = [&](int v) __attribute__((always_inline)) {
+            auto smallest = [](int x) __attribute__((always_inline)) {
+                x = min(x, xor_lane<1>(x));
+                x = min(x, xor_lane<2>(x));
+                x = min(x, xor_lane<4>(x));
+                if constexpr (W > 8) x = min(x, xor_lane<8>(x));
+                return x;
+            };
+            const int low = smallest(v);
+            const int at = __ffsll(static_cast<unsigned long long>(__builtin_amdgcn_ballot_w64(v == low))) - 1;
+            return smallest(lane % W == at ? 0x7f800000 : v);
+        };
+        // One granule step with abandoned tiles. next_heads: the granule's head codes, loaded a step ahead; dword u of
+        // next_heads[h] holds codes 4h .. 4h + 3 of tile u.
+        uint4 next_heads[kPrune ? kHeadWords : 1];
+        unsigned global_raw = 0;  // first wave: the slab's shared bounds as last read (complemented bits, 0: none)
+        const bool exchange = wave == 0 && shared_bounds != nullptr;
+        auto load_heads = [&](int64_t at) __attribute__((always_inline)) {
+            const uint4* c = a.heads + at * (kHeadWords * WAVE) + lane;
+#pragma unroll
+            for (int h = 0; h < kHeadWords; ++h) next_heads[h] = c[h * WAVE];
+        };
+        constexpr int WORDS = M ? M / 16 : 1;
+        constexpr int kShift = log2_int(E::kBytes);
+        // Entry group of sub-space s for its code byte in `part`.
+        auto read = [&](auto sc, uint32_t part) __attribute__((always_inline)) -> V {
+            constexpr int s = decltype(sc)::value, j = s % 16, base = s * KSUB * E::kBytes;
+            uint32_t reg;
+            int imm;
+            if constexpr ((base >> 16) == 0) {
+                reg = scaled_byte<kShift>(part, j & 3);
+                imm = base;
+            } else {
+                scaled_byte_low_half<kShift, j & 3>(hi[j % kHi], part);
+                reg = hi[j % kHi];
+                imm = base - 65536;
+            }
+            return *reinterpret_cast<const V*>(tables + reg + imm);
+        };
+        auto word_part = [](const uint4& w, int j) __attribute__((always_inline)) {
+            return j < 4 ? w.x : j < 8 ? w.y : j < 12 ? w.z : w.w;
+        };
+        // Sub-spaces [S0, S1) of one tile, in batches of eight reads issued before their adds; the first sub-space sets
+        // the sums. code(s): the dword that holds the code byte of sub-space s.
+        auto span = [&](auto s0c, auto s1c, auto&& code, float* acc) __attribute__((always_inline)) {
+            constexpr int S0 = decltype(s0c)::value, S1 = decltype(s1c)::value;
+            static_for<0, (S1 - S0 + 7) / 8>([&](auto bc) {
+                constexpr int b0 = S0 + decltype(bc)::value * 8;
+                constexpr int count = S1 - b0 < 8 ? S1 - b0 : 8;
+                V v[8];
+                static_for<0, count>([&](auto jc) {
+                    constexpr int s = b0 + decltype(jc)::value;
+                    v[decltype(jc)::value] = read(std::integral_constant<int, s>{}, code(s));
+                });
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int jj = 0; jj < count; ++jj) {
+                    if (b0 == 0 && jj == 0) E::set(acc, v[jj]);
+                    else E::add(acc, v[jj], one);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        // Bounds before the scan. Until a block has met vectors near a query no tile can be dropped for it, and with
+        // four queries a block would sum a thousand-odd tiles in full before it has met all four's neighbourhoods. So
+        // each wave first compares one vector of every tile of its share by the first kCheck sub-spaces, 64 tiles at a
+        // time, and sums the best tile of each query: the tile's K-th smallest distance is that of K real vectors (K >
+        // 64: the ceil(K/2)-th of two waves' tiles).
+        auto first_bounds = [&]() __attribute__((always_inline)) {
+            float best[QS];
+            uint32_t best_tile[QS];
+#pragma unroll
+            for (int q = 0; q < QS; ++q) {
+                best[q] = INFINITY;
+                best_tile[q] = 0xffffffffu;
+            }
+            const uint32_t end_tile = static_cast<uint32_t>(min<int64_t>(g_hi * U, (a.n + WAVE - 1) / WAVE));
+            const uint32_t* const head_words = reinterpret_cast<const uint32_t*>(a.heads);
+            for (uint32_t t0 = static_cast<uint32_t>(g_lo * U) + wave * WAVE; t0 < end_tile; t0 += W * WAVE) {
+                const uint32_t tile = min(t0 + static_cast<uint32_t>(lane), end_tile - 1);
+                uint32_t part[kHeadWords];
+#pragma unroll
+                for (int h = 0; h < kHeadWords; ++h)
+                    part[h] = head_words[(static_cast<int64_t>(tile >> 2) * kHeadWords + h) * (WAVE * 4) + (tile & 3)];
+                float sum[QS];
+                span(std::integral_constant<int, 0>{}, std::integral_constant<int, kCheck>{},
+                     [&](int s) __attribute__((always_inline)) { return part[s / 4]; }, sum);
+#pragma unroll
+                for (int q = 0; q < QS; ++q) {
+                    const bool nearer = sum[q] < best[q];
+                    best[q] = nearer ? sum[q] : best[q];
+                    best_tile[q] = nearer ? tile : best_tile[q];
+                }
+            }
+            const int rank = (kHalfRank && a.K > WAVE ? (a.K + 1) / 2 : a.K) - 1;
+#pragma unroll 1
+            for (int i = 0; i < QS; ++i) {  // one copy of the sums and the sort
+                uint64_t key = 0;
+                static_for<0, QS>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    if (i == q) key = (static_cast<uint64_t>(__float_as_uint(best[q])) << 32) | best_tile[q];
+                });
+                auto nearest = [&](auto jc) __attribute__((always_inline)) {
+                    constexpr int j = decltype(jc)::value;
+                    const uint64_t other = static_cast<uint64_t>(
+                        (static_cast<uint64_t>(static_cast<uint32_t>(xor_lane<j>(static_cast<int>(key >> 32)))) << 32) |
+                        static_cast<uint32_t>(xor_lane<j>(static_cast<int>(static_cast<uint32_t>(key)))));
+                    key = other < key ? other : key;
+                };
+                nearest(std::integral_constant<int, 1>{});
+                nearest(std::integral_constant<int, 2>{});
+                nearest(std::integral_constant<int, 4>{});
+                nearest(std::integral_constant<int, 8>{});
+                nearest(std::integral_constant<int, 16>{});
+                nearest(std::integral_constant<int, 32>{});
+                const uint32_t tile = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(key)));
+                if (tile >= end_tile) continue;  // no tile in this wave's share, or no finite sum
+                uint4 cw[WORDS];
+#pragma unroll
+                for (int w = 0; w < WORDS; ++w) cw[w] = a.codes[(static_cast<int64_t>(tile) * WORDS + w) * WAVE + lane];
+                float sum[QS];
+                span(std::integral_constant<int, 0>{}, std::integral_constant<int, M>{},
+                     [&](int s) __attribute__((always_inline)) { return word_part(cw[s / 16], s % 16); }, sum);
+                uint32_t mine = 0;
+                static_for<0, QS>([&](auto qc) {
+                    if (i == decltype(qc)::value) mine = __float_as_uint(sum[decltype(qc)::value]);
+                });
+                // No distance where the tile is past the end, and NaN (any bits above infinity's) as infinity.
+                if (tile * WAVE + static_cast<uint32_t>(lane) >= n32) mine = 0x7f800000u;
+                uint64_t sorted = (static_cast<uint64_t>(min(mine, 0x7f800000u)) << 32) | static_cast<uint32_t>(lane);
+                wave_sort<2, false>(sorted);
+                const uint32_t bound = static_cast<uint32_t>(
+                    __builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(sorted >> 32)), rank));
+                if constexpr (kHalfRank) {
+                    if (a.K > WAVE) half_rank[i][wave] = static_cast<int>(bound);
+                    else atomicMin(&block_bound[i], bound);
+                } else {
+                    atomicMin(&block_bound[i], bound);
+                }
+            }
+            __syncthreads();
+            if constexpr (kHalfRank) {
+                if (a.K > WAVE) {
+#pragma unroll 1
+                    for (int i = 0; i < QS; ++i)
+                        atomicMin(&block_bound[i], static_cast<unsigned>(second_smallest(half_rank[i][lane % W])));
+                }
+            }
+        };
+        auto prune_step = [&]() __attribute__((always_inline)) {
+            constexpr int kHalf = M / 2;
+            unsigned grab = 0;
+            if (lane == 0) grab = atomicAdd(&next_gran, 1u);
+            // Lane l holds query l % QS's bound (no lane is masked off: the scan's control flow stays wave-uniform).
+            unsigned bound_raw = block_bound[lane % QS];
+            const int64_t tile0 = g * U;
+            const uint4* tile_codes = a.codes + tile0 * WORDS * WAVE + lane;
+            uint4 heads[kHeadWords];
+#pragma unroll
+            for (int h = 0; h < kHeadWords; ++h) heads[h] = next_heads[h];
+            if (g_ahead < g_hi) load_heads(g_ahead);
+            // The slab's blocks exchange bounds through their first waves.
+            if (exchange) {  // wave-uniform
+                const unsigned other = ~global_raw;
+                if (__builtin_amdgcn_ballot_w64(other < bound_raw)) atomicMin(&block_bound[lane % QS], other);
+                if (__builtin_amdgcn_ballot_w64(bound_raw < other && bound_raw < 0x7f800000u)) {
+                    if (lane < QS)
+                        __hip_atomic_fetch_max(shared_bounds + lane, ~bound_raw, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+                }
+                bound_raw = min(bound_raw, other);
+                global_raw = __hip_atomic_load(shared_bounds + lane % QS, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+            }
+            float f[QS];  // admission bounds, wave-uniform (-inf for padded query slots)
+#pragma unroll
+            for (int q = 0; q < QS; ++q)
+                f[q] = __int_as_float(min(__float_as_int(lists[q].filter),
+                                          __builtin_amdgcn_readlane(static_cast<int>(bound_raw), q)));
+            auto alive = [&](const float* acc) __attribute__((always_inline)) {
+                uint64_t any = 0;
+#pragma unroll
+                for (int q = 0; q < QS; ++q) any |= __builtin_amdgcn_ballot_w64(acc[q] <= f[q]);
+                return any != 0;
+            };
+            // The first kCheck sub-spaces of the four tiles, eight reads in flight at a time.
+            auto head_part = [&](int u, int h) __attribute__((always_inline)) {
+                return u == 0 ? heads[h].x : u == 1 ? heads[h].y : u == 2 ? heads[h].z : heads[h].w;
+            };
+            float acc[U][QS];
+            static_for<0, (kCheck + 3) / 4>([&](auto bc) {
+                constexpr int s0 = decltype(bc)::value * 4, width = kCheck - s0 < 4 ? kCheck - s0 : 4;
+                constexpr int group = 8 / width;  // tiles per batch
+                static_for<0, U / group>([&](auto gc) {
+                    constexpr int u0 = decltype(gc)::value * group;
+                    V v[group][width];
+                    static_for<0, group>([&](auto uc) {
+                        static_for<0, width>([&](auto jc) {
+                            constexpr int s = s0 + decltype(jc)::value;
+                            v[decltype(uc)::value][decltype(jc)::value] =
+                                read(std::integral_constant<int, s>{}, head_part(u0 + decltype(uc)::value, s / 4));
+                        });
+                    });
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int u = 0; u < group; ++u)
+#pragma unroll
+                        for (int jj = 0; jj < width; ++jj) {
+                            if (s0 == 0 && jj == 0) E::set(acc[u0 + u], v[u][jj]);
+                            else E::add(acc[u0 + u], v[u][jj], one);
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            });
+            unsigned live_tiles = 0;  // wave-uniform
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (alive(acc[u])) live_tiles |= 1u << u;
+            bool changed = false;
+            // The tiles that may hold candidates, one at a time (one copy of the code: their codes and sums are moved
+            // into place by a wave-uniform branch).
+            while (live_tiles) {
+                const int u = __ffs(static_cast<int>(live_tiles)) - 1;
+                live_tiles &= live_tiles - 1;
+                float sum[QS];
+                uint32_t part[kHeadWords];
+                static_for<0, U>([&](auto uc) {
+                    if (u == decltype(uc)::value) {
+#pragma unroll
+                        for (int h = 0; h < kHeadWords; ++h) part[h] = head_part(decltype(uc)::value, h);
+#pragma unroll
+                        for (int q = 0; q < QS; ++q) sum[q] = acc[decltype(uc)::value][q];
+                    }
+                });
+                auto head_code = [&](int s) __attribute__((always_inline)) { return part[s / 4]; };
+                if constexpr (kCheck < kHeadBytes) {
+                    span(std::integral_constant<int, kCheck>{}, std::integral_constant<int, kHeadBytes>{}, head_code, sum);
+                    if (!alive(sum)) continue;
+                }
+                uint4 cw[WORDS];
+                auto word_code = [&](int s) __attribute__((always_inline)) { return word_part(cw[s / 16], s % 16); };
+                const uint4* words_u = tile_codes + u * (WORDS * WAVE);
+                constexpr int kFirstWord = kHeadBytes / 16, kHalfWords = (kHalf + 15) / 16;
+                if constexpr (kHalf > kHeadBytes) {
+#pragma unroll
+                    for (int w = kFirstWord; w < kHalfWords; ++w) cw[w] = words_u[w * WAVE];
+                    span(std::integral_constant<int, kHeadBytes>{}, std::integral_constant<int, kHalf>{}, word_code, sum);
+                    if (!alive(sum)) continue;
+                }
+                constexpr int kRest = kHalf > kHeadBytes ? kHalf : kHeadBytes;  // sub-spaces summed so far
+#pragma unroll
+                for (int w = kHalf > kHeadBytes ? kHalfWords : kFirstWord; w < WORDS; ++w) cw[w] = words_u[w * WAVE];
+                span(std::integral_constant<int, kRest>{}, std::integral_constant<int, M>{}, word_code, sum);
+                if (!alive(sum)) continue;
+                const int64_t tile = tile0 + u;
+                const uint32_t first = static_cast<uint32_t>(tile * WAVE);
+                const int32_t id = static_cast<int32_t>(a.slot_ids[(tile >> 2) * 256 + lane * 4 + (tile & 3)]);
+                const uint64_t valid =
+                    first + WAVE <= n32 ? ~uint64_t{0}
+                                        : __builtin_amdgcn_ballot_w64(first + static_cast<uint32_t>(lane) < n32);
+#pragma unroll
+                for (int q = 0; q < QS; ++q) {
+                    const uint64_t mask = __builtin_amdgcn_ballot_w64(sum[q] <= f[q]) & valid;
+                    if (!mask) continue;
+                    if constexpr (kQueue) queue_offer(q, sum[q], id, mask);
+                    else lists[q].offer_masked_bulk(sum[q], id, mask, a.K);
+                    f[q] = __int_as_float(min(__float_as_int(f[q]), __float_as_int(lists[q].filter)));
+                }
+                changed = true;
+            }
+            if constexpr (kHalfRank) {
+                if (changed) {
+                    const int rank = (a.K + 1) / 2 - 1;  // < 64: in the lists' first register
+#pragma unroll
+                    for (int q = 0; q < QS; ++q) {
+                        half_rank[q][wave] = __float_as_int(lane_read(lists[q].d[0], rank));
+                        f[q] = __int_as_float(min(__float_as_int(f[q]), second_smallest(half_rank[q][lane % W])));
+                    }
+                }
+            }
+            if (changed) {  // publish this wave's K-th best distances
+                int pub = 0;
+#pragma unroll
+                for (int q = 0; q < QS; ++q) pub = lane % QS == q ? __float_as_int(kHalfRank ? f[q] : lists[q].thr_d) : pub;
+                atomicMin(&block_bound[lane % QS], static_cast<unsigned>(pub));
+            }
+            g = g_ahead;
+            g_ahead = g_lo + static_cast<int64_t>(__builtin_amdgcn_readfirstlane(grab));
+        };
         // Lists that admit one by one take a wave's first step in bulk: the fresh lists admit about a third of the
         // first tile's candidates and, one by one, those inserts made the step several times a later one, with
         // every wave of the CU inserting at once. The step is a separate copy of the body ahead of the loop, so the
         // loop's own code is that of one-by-one admission (1M x nq=1000: -1.2 %; fp16 tables, 8 queries: -5 %).
-        constexpr bool kPeel = !(IVF || S > 1 || kBulkOne || BULK);
+        constexpr bool kPeel = !(IVF || S > 1 || kBulkOne || BULK || kPrune);
         if constexpr (kPeel) {
             if (g < g_hi) granule(std::true_type{});
         }
-        while (g < g_hi) granule(std::false_type{});
+        if constexpr (kPrune) {
+            first_bounds();
+            if (g < g_hi) load_heads(g);
+            while (g < g_hi) prune_step();
+        } else {
+            while (g < g_hi) granule(std::false_type{});
+        }
         // Queued candidates go into the lists before they are stored (inverted lists: at the end of a query's run).
         auto flush_all = [&]() __attribute__((always_inline)) {
             if constexpr (kQueue) {
@@ -1087,9 +1414,8 @@ __global__ void __launch_bounds__(T)
         // Partial lists of this (block, slab): part[slab][q][slot][list][K], the lists of one query contiguous.
         // With few blocks per slab every wave writes its own lists; with many, the block first merges its W lists
         // per query in LDS (the tables are dead by then), so the final merge reads W times fewer pairs.
-        const int64_t lo = first_block_of(slab_first, grid, total);
-        const int count = static_cast<int>(first_block_of(slab_next - 1, grid, total) - lo + 1);
-        const int slot = static_cast<int>(b - lo);
+        const int count = slab_blocks;
+        const int slot = static_cast<int>(b - slab_lo);
         const int lpb = a.lists_per_block;
         const int slots = a.max_slots;  // every slab reserves max_slots blocks
         Pair* const slab_part = a.part + slab * QS * a.max_slots * lpb * static_cast<int64_t>(a.K);
@@ -1142,6 +1468,9 @@ __global__ void __launch_bounds__(T)
         __syncthreads();
         if (last_block) {
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            // Every block of the slab has finished with the shared bounds: back to zero for the next search.
+            if (shared_bounds && tid < QS)
+                __hip_atomic_store(shared_bounds + tid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (lpb == W || QS > 1) {  // one wave per query, the queries in parallel
                 const int per_block = lpb == W ? W : 1;
                 for (int q = wave; q < QS && slab * QS + q < a.nq; q += W)
@@ -1156,20 +1485,21 @@ __global__ void __launch_bounds__(T)
     }
 }
 
-template <int QG, int NG, int U, int M, int S, int T, bool F16, bool IVF, bool BULK>
+template <int QG, int NG, int U, int M, int S, int T, bool F16, bool IVF, bool BULK, bool ABANDON>
 hipError_t launch_fused_wave_t(const WaveScanArgs& a, int grid, size_t smem, hipStream_t stream) {
-    hipLaunchKernelGGL((fused_wave_kernel_t<QG, NG, U, M, S, T, F16, IVF, BULK>), dim3(grid), dim3(T), smem, stream,
-                       a);
+    hipLaunchKernelGGL((fused_wave_kernel_t<QG, NG, U, M, S, T, F16, IVF, BULK, ABANDON>), dim3(grid), dim3(T), smem,
+                       stream, a);
     return hipGetLastError();
 }
 
-template <int QG, int NG, int U, int M, int S, bool F16, bool IVF = false, bool BULK = false, int T = 512>
+template <int QG, int NG, int U, int M, int S, bool F16, bool IVF = false, bool BULK = false, int T = 512,
+          bool ABANDON = false>
 WaveScanKernel make_wave_kernel() {
     WaveScanKernel k;
-    k.fn = reinterpret_cast<const void*>(&fused_wave_kernel_t<QG, NG, U, M, S, T, F16, IVF, BULK>);
+    k.fn = reinterpret_cast<const void*>(&fused_wave_kernel_t<QG, NG, U, M, S, T, F16, IVF, BULK, ABANDON>);
     k.threads = T;
     k.dynamic_lds = M == 0;
-    k.launch = &launch_fused_wave_t<QG, NG, U, M, S, T, F16, IVF, BULK>;
+    k.launch = &launch_fused_wave_t<QG, NG, U, M, S, T, F16, IVF, BULK, ABANDON>;
     return k;
 }
 
@@ -1237,6 +1567,34 @@ WaveScanKernel select_wave_kernel(int qg, int ng, int ilp, int segments, bool bu
     }
 #undef VK_WAVE_CASE
 #undef VK_WAVE_ILP
+    return WaveScanKernel{};
+}
+
+// Instances that abandon tiles, for one M and entry type: one table group, four tiles per wave step, 1024-thread blocks
+// where kWideBlock holds (more waves share a bound), else 512.
+template <int M, bool F16>
+WaveScanKernel select_abandon_kernel(int q, int segments, int threads) {
+    constexpr int kLds = 160 * 1024;
+#define VK_ABANDON(QG_, S_)                                                                                       \
+    if (q == QG_ && segments == S_) {                                                                            \
+        if constexpr (M * KSUB * Entries<QG_, F16>::kBytes <= kLds) {                                             \
+            if constexpr (kWideBlock<QG_, 1, M, S_, F16>) {                                                      \
+                if (threads == 1024) return make_wave_kernel<QG_, 1, 4, M, S_, F16, false, false, 1024, true>(); \
+            }                                                                                                    \
+            if (threads == 512) return make_wave_kernel<QG_, 1, 4, M, S_, F16, false, false, 512, true>();       \
+        }                                                                                                        \
+    }
+    VK_ABANDON(1, 1)
+    VK_ABANDON(1, 2)
+    VK_ABANDON(2, 1)
+    VK_ABANDON(2, 2)
+    VK_ABANDON(4, 1)
+    VK_ABANDON(4, 2)
+    if constexpr (F16) {
+        VK_ABANDON(8, 1)
+        VK_ABANDON(8, 2)
+    }
+#undef VK_ABANDON
     return WaveScanKernel{};
 }
 

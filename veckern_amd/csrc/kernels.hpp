@@ -23,6 +23,14 @@ hipError_t launch_build_words(const uint8_t* codes, int64_t n, int m, int64_t n_
 // [n, n_pad) are zero.
 hipError_t launch_build_sorted_words(const uint8_t* codes, int64_t n, int m, int64_t n_pad, const uint32_t* slot_ids,
                                      const uint8_t* rows, uint4* out, hipStream_t stream);
+// The head codes of a word-interleaved layout, the first 4 * head_words codes of every vector by granules of four tiles:
+// out[(granule * head_words + h) * 64 + lane], dword u = codes 4h .. 4h + 3 of the vector in tile 4 * granule + u.
+hipError_t launch_build_heads(const uint4* words, int m, int64_t n_pad, int head_words, uint4* out, hipStream_t stream);
+inline int abandon_head_words(int m) { return m <= 32 ? 2 : m / 16; }
+// sums[0] += the squared distances between the codewords of neighbouring slots' vectors (lane ^ 1), sums[1] += those
+// between vectors half the database apart, over the sub-spaces past the fourth and every `stride`-th tile.
+hipError_t launch_tile_spread(const uint8_t* codes, const uint32_t* slot_ids, const float* centroids, int m, int dsub,
+                              int64_t tiles, int64_t stride, double* sums, hipStream_t stream);
 // Byte-interleaved: out[(tile * m + s) * 64 + lane] = sub-code s of vector tile*64+lane.
 hipError_t launch_build_bytes(const uint8_t* codes, int64_t n, int m, int64_t n_pad, uint8_t* out,
                               hipStream_t stream);
@@ -62,6 +70,10 @@ struct WaveScanArgs {
     int lists_per_block;     // partial lists a block writes per (slab, query): one per wave, or 1 (merged in LDS)
     Pair* part;              // [slabs][qg * ng][max_slots][lists_per_block][K]
     unsigned* counters;      // [slabs], zero between searches: blocks of a slab that have finished
+    // [slabs][qg * ng], zero between searches, or nullptr: per query the smallest K-th best distance that a block of
+    // the slab has found, as complemented raw bits (so that zero means none and the largest word wins).
+    unsigned* bounds;
+    const uint4* heads;      // head codes (launch_build_heads) for the instances that abandon tiles
     Pair* out;               // [nq][k]; empty slots become {+inf, -1}
     // Inverted lists (IVF instances only, one query per slab, the plan of launch_ivf_plan); `n_gran`, `total` and
     // `max_slots` are then unused (the total is query_gran[nq]).
@@ -81,6 +93,9 @@ struct WaveScanKernel {
     hipError_t (*launch)(const WaveScanArgs&, int grid, size_t smem, hipStream_t) = nullptr;
 };
 
+// The instance that abandons tiles (m = 16, 32, 48, 64; q queries in one table group; 1024 or 512 threads); fn ==
+// nullptr when it is not built.
+WaveScanKernel abandon_kernel(int q, int m, int segments, bool f16, int threads);
 // Returns a kernel with fn == nullptr when the combination is not built. f16: binary16 tables (v9). bulk: the
 // instance with bulk admission into one-register lists (fp32, more than one query per block only). threads: block
 // size, 512 or 1024 (built for four tiles per wave step where two 512-thread blocks' tables fit one CU).

@@ -100,4 +100,69 @@ hipError_t launch_zero_words(unsigned* p, int64_t count, hipStream_t stream) {
     return hipGetLastError();
 }
 
+namespace {
+
+__global__ void build_heads_kernel(const uint32_t* words, int m, int64_t granules, int head_words, uint4* out) {
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;  // (granule, h, lane)
+    if (e >= granules * head_words * WAVE) return;
+    const int lane = static_cast<int>(e % WAVE), h = static_cast<int>(e / WAVE % head_words);
+    const int64_t tile0 = e / WAVE / head_words * 4;
+    auto part = [&](int u) {
+        return words[(((tile0 + u) * (m / 16) + h / 4) * WAVE + lane) * 4 + h % 4];
+    };
+    out[e] = make_uint4(part(0), part(1), part(2), part(3));
+}
+
+// One block per sampled tile of the slot order: squared distances between the codewords of neighbouring lanes' vectors,
+// and of each lane's vector and one half the database away, over the sub-spaces past the sort key.
+__global__ void __launch_bounds__(WAVE)
+    tile_spread_kernel(const uint8_t* codes, const uint32_t* slot_ids, const float* centroids, int m, int dsub,
+                       int64_t tiles, int64_t stride, double* sums) {
+    const int64_t tile = static_cast<int64_t>(blockIdx.x) * stride, far_tile = (tile + tiles / 2) % tiles;
+    const int lane = threadIdx.x;
+    auto row = [&](int64_t t, int l) {
+        return codes + static_cast<int64_t>(slot_ids[(t >> 2) * 256 + l * 4 + (t & 3)]) * m;
+    };
+    const uint8_t* const own = row(tile, lane);
+    const uint8_t* const next = row(tile, lane ^ 1);
+    const uint8_t* const other = row(far_tile, lane);
+    float close = 0.f, apart = 0.f;
+    for (int s = 4; s < m; ++s) {
+        const float* c = centroids + static_cast<int64_t>(s) * KSUB * dsub;
+        for (int j = 0; j < dsub; ++j) {
+            const float x = c[own[s] * dsub + j], dn = x - c[next[s] * dsub + j], df = x - c[other[s] * dsub + j];
+            close += dn * dn;
+            apart += df * df;
+        }
+    }
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) {
+        close += __shfl_xor(close, o);
+        apart += __shfl_xor(apart, o);
+    }
+    if (lane == 0) {
+        atomicAdd(&sums[0], static_cast<double>(close));
+        atomicAdd(&sums[1], static_cast<double>(apart));
+    }
+}
+
+}  // namespace
+
+hipError_t launch_build_heads(const uint4* words, int m, int64_t n_pad, int head_words, uint4* out,
+                              hipStream_t stream) {
+    const int64_t granules = n_pad / 256, threads = granules * head_words * WAVE;
+    hipLaunchKernelGGL(build_heads_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream,
+                       reinterpret_cast<const uint32_t*>(words), m, granules, head_words, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_tile_spread(const uint8_t* codes, const uint32_t* slot_ids, const float* centroids, int m, int dsub,
+                              int64_t tiles, int64_t stride, double* sums, hipStream_t stream) {
+    const int64_t blocks = (tiles + stride - 1) / stride;
+    if (blocks <= 0) return hipSuccess;
+    hipLaunchKernelGGL(tile_spread_kernel, dim3(static_cast<unsigned>(blocks)), dim3(WAVE), 0, stream, codes, slot_ids,
+                       centroids, m, dsub, tiles, stride, sums);
+    return hipGetLastError();
+}
+
 }  // namespace vk
