@@ -36,10 +36,10 @@ def fixture(family, n, d, m, nq):
 @pytest.mark.parametrize("family", ["clusters", "uniform", "ties", "overflow"])
 @pytest.mark.parametrize("d,m", [(64, 16), (64, 32), (96, 48), (128, 64)])
 def test_abandoned_tiles_match_oracle(family, d, m):
-    n, nq = 40_003, 21
+    n, nq = 140_003, 21  # at 1 to 4 blocks per slab, enough vectors per block for these scans
     cent, codes, queries = fixture(family, n, d, m, nq)
     with vk.PQSearcher(cent, codes, d) as s:
-        for q, threads, blocks in [(1, 256, 0), (2, 1024, 0), (4, 512, 1), (4, 256, 16), (8, 1024, 3)]:
+        for q, threads, blocks in [(1, 256, 4), (2, 1024, 2), (4, 512, 1), (4, 256, 3), (8, 1024, 3), (4, 256, 0)]:
             s.set_tuning(vk.Tuning(queries_per_block=q, scan_threads=threads, blocks_per_query=blocks))
             for k, count in [(1, nq), (10, 1), (64, 5), (100, nq)]:
                 got_d, got_i, _ = s.search(queries[:count], k, V8)
@@ -62,7 +62,7 @@ def test_single_query_over_many_blocks_repeats():
     cent, codes, queries = datagen.pq_fixture(600_000, 64, 16, 4, seed=920)
     exp = orc.adc_search(cent, 64, codes, queries, 10)
     with vk.PQSearcher(cent, codes, 64) as s:
-        s.set_tuning(vk.Tuning(queries_per_block=4))
+        s.set_tuning(vk.Tuning(queries_per_block=4, blocks_per_query=12))
         for r in range(12):  # each search starts without the bounds of the one before
             q = r % 4
             got_d, got_i, _ = s.search(queries[q:q + 1], 10, V8)

@@ -35,21 +35,21 @@ WaveScanKernel fused_wave_kernel_h48(int qg, int ng, int ilp, int segments, bool
 WaveScanKernel fused_wave_kernel_h64(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_hx(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 
-WaveScanKernel abandon_kernel_m16(int q, int segments, int threads);
-WaveScanKernel abandon_kernel_m32(int q, int segments, int threads);
-WaveScanKernel abandon_kernel_m48(int q, int segments, int threads);
-WaveScanKernel abandon_kernel_m64(int q, int segments, int threads);
-WaveScanKernel abandon_kernel_h16(int q, int segments, int threads);
-WaveScanKernel abandon_kernel_h32(int q, int segments, int threads);
-WaveScanKernel abandon_kernel_h48(int q, int segments, int threads);
-WaveScanKernel abandon_kernel_h64(int q, int segments, int threads);
+WaveScanKernel abandon_kernel_m16(int q, int threads);
+WaveScanKernel abandon_kernel_m32(int q, int threads);
+WaveScanKernel abandon_kernel_m48(int q, int threads);
+WaveScanKernel abandon_kernel_m64(int q, int threads);
+WaveScanKernel abandon_kernel_h16(int q, int threads);
+WaveScanKernel abandon_kernel_h32(int q, int threads);
+WaveScanKernel abandon_kernel_h48(int q, int threads);
+WaveScanKernel abandon_kernel_h64(int q, int threads);
 
-WaveScanKernel abandon_kernel(int q, int m, int segments, bool f16, int threads) {
+WaveScanKernel abandon_kernel(int q, int m, bool f16, int threads) {
     switch (m) {
-        case 16: return f16 ? abandon_kernel_h16(q, segments, threads) : abandon_kernel_m16(q, segments, threads);
-        case 32: return f16 ? abandon_kernel_h32(q, segments, threads) : abandon_kernel_m32(q, segments, threads);
-        case 48: return f16 ? abandon_kernel_h48(q, segments, threads) : abandon_kernel_m48(q, segments, threads);
-        case 64: return f16 ? abandon_kernel_h64(q, segments, threads) : abandon_kernel_m64(q, segments, threads);
+        case 16: return f16 ? abandon_kernel_h16(q, threads) : abandon_kernel_m16(q, threads);
+        case 32: return f16 ? abandon_kernel_h32(q, threads) : abandon_kernel_m32(q, threads);
+        case 48: return f16 ? abandon_kernel_h48(q, threads) : abandon_kernel_m48(q, threads);
+        case 64: return f16 ? abandon_kernel_h64(q, threads) : abandon_kernel_m64(q, threads);
         default: return WaveScanKernel{};
     }
 }
@@ -439,19 +439,10 @@ struct vk_searcher {
         // fp32: 8 queries are two groups of 4 (16-byte reads); fp16: up to 8 queries in one group.
         const int qg = (!f16 && w.q == 8) ? 4 : w.q, ng = (!f16 && w.q == 8) ? 2 : 1;
         w.ilp = tuning.vectors_per_step;
-        bool abandon = false;
-        if (abandon_tiles && w.ilp == 4 && ng == 1) {
-            if (tuning.scan_threads != 512)
-                w.kern = vk::abandon_kernel(w.q, static_cast<int>(m), segments, f16, 1024);
-            if (!w.kern.fn) w.kern = vk::abandon_kernel(w.q, static_cast<int>(m), segments, f16, 512);
-            abandon = w.kern.fn != nullptr;
-        }
-        if (!abandon) w.kern = vk::fused_wave_kernel(qg, ng, w.ilp, static_cast<int>(m), segments, f16);
-        if (!w.kern.fn) fail(VK_ERR_LOGIC, "no fused-warp kernel built for this (Q, ILP, m, K)");
         const size_t tables = static_cast<size_t>(w.q) * m * vk::KSUB * entry_bytes;
         require(tables <= info.max_smem_per_block, "LUT does not fit in LDS");
-        w.smem = w.kern.dynamic_lds ? tables : 0;  // fixed-m instances hold the tables in static LDS
         auto plan_for = [&](const vk::WaveScanKernel& k) {
+            w.smem = k.dynamic_lds ? tables : 0;  // fixed-m instances hold the tables in static LDS
             if (k.dynamic_lds)
                 VK_HIP(hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(w.smem)));
             VK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&w.per_cu, k.fn, k.threads, w.smem));
@@ -460,7 +451,20 @@ struct vk_searcher {
                                                   static_cast<int64_t>(w.per_cu) * info.sm_count,
                                                   tuning.blocks_per_query, info.sm_count);
         };
-        plan_for(w.kern);
+        bool abandon = false;
+        if (abandon_tiles && w.ilp == 4 && ng == 1 && segments == 1) {
+            vk::WaveScanKernel k;
+            if (tuning.scan_threads != 512) k = vk::abandon_kernel(w.q, static_cast<int>(m), f16, 1024);
+            if (!k.fn) k = vk::abandon_kernel(w.q, static_cast<int>(m), f16, 512);
+            if (k.fn) {
+                w.kern = k;
+                plan_for(w.kern);
+                abandon = vk::plan::block_vectors(w.part, w.ilp) >= vk::plan::kAbandonVectors;
+            }
+        }
+        if (!abandon) w.kern = vk::fused_wave_kernel(qg, ng, w.ilp, static_cast<int>(m), segments, f16);
+        if (!w.kern.fn) fail(VK_ERR_LOGIC, "no fused-warp kernel built for this (Q, ILP, m, K)");
+        if (!abandon) plan_for(w.kern);
         // 1024-thread blocks where that instance exists and its blocks scan many vectors of their slabs (above the
         // bulk-scan bound; and not crossing slab boundaries where 512-thread blocks would not): one block per CU,
         // whose 16 waves share one granule counter, instead of two 512-thread blocks that the CU does not balance

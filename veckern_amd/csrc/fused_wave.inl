@@ -610,8 +610,8 @@ __global__ void __launch_bounds__(T)
     // by any query. Entries are sums of squares, so a running sum never falls (rounding to nearest is monotone): a
     // partial sum beyond the bound means a distance beyond it, and a NaN stays a NaN, which no list admits. The bound
     // of a query is the smallest of
-    //  - the K-th best distance of any wave's list in the block, and for K > 64 the second smallest of the waves'
-    //    ceil(K/2)-th best (two waves then hold K candidates at or below it), in block_bound;
+    //  - the K-th best distance of any wave's list in the block, and the bounds found before the scan (first_bounds), in
+    //    block_bound;
     //  - where several blocks share a slab, the bounds of its other blocks (a.bounds).
     // K real candidates lie at or below it, so nothing beyond it reaches the merged top K; ties at it are kept.
     // In the sorted slot order a tile's vectors are alike, so they fail together: on the 1M-vector Gaussian mixture 98 %
@@ -619,15 +619,14 @@ __global__ void __launch_bounds__(T)
     // The first kHeadBytes codes of every vector are read from an array of their own (a.heads): the scan reads half of
     // the code bytes at m = 16 and a quarter at m = 32 .. 64, the rest and the ids only for tiles that are left.
     constexpr bool kPrune = ABANDON;
-    static_assert(!ABANDON || (M > 0 && M <= 64 && U == 4 && NG == 1 && !IVF && !BULK), "instances that abandon tiles");
+    static_assert(!ABANDON || (M > 0 && M <= 64 && U == 4 && S == 1 && NG == 1 && !IVF && !BULK), "instances that abandon tiles");
     constexpr int kHeadWords = M <= 32 ? 2 : M / 16;  // dwords per vector
     constexpr int kHeadBytes = 4 * kHeadWords;
     // The first check: a quarter of the sub-spaces; at m = 16 a quarter lets a third of the tiles of four queries
     // through, two more sub-spaces (10 VALU per tile) stop nearly all of those.
     constexpr int kCheck = M == 16 && QS >= 4 ? 6 : M / 4;
     __shared__ unsigned block_bound[QS];  // raw bits of a distance >= 0 or +inf: unsigned order is float order
-    constexpr bool kHalfRank = kPrune && S > 1;
-    __shared__ int half_rank[kHalfRank ? QS : 1][W];  // raw bits of the waves' ceil(K/2)-th best
+    __shared__ int share_rank[kPrune ? QS : 1][W];  // raw bits of the ceil(K/W)-th best of each wave's best tile
     // Long lists (K > 64), and the bulk instances (few vectors per block): per (query, wave), the distance of the
     // wave list's entry ceil(K/W) - 1 for the current slab (raw bits of a distance >= 0, so unsigned order is float
     // order; +inf until the list holds that many). If every wave holds ceil(K/W) entries at or below T, the block
@@ -796,8 +795,8 @@ __global__ void __launch_bounds__(T)
                 for (int t = tid; t < QS * W; t += T) (&rank_bound[0][0])[t] = 0x7f800000u;  // +inf
             if (!IVF && tid == 0) next_gran = kPrune ? 2 * W : W;
             if (kPrune && tid < QS) block_bound[tid] = 0x7f800000u;  // +inf
-            if constexpr (kHalfRank)
-                for (int t = tid; t < QS * W; t += T) (&half_rank[0][0])[t] = 0x7f800000;
+            if constexpr (kPrune)
+                for (int t = tid; t < QS * W; t += T) (&share_rank[0][0])[t] = 0x7f800000;
             __syncthreads();
 
             // A padded query slot (past nq in the last slab) gets the threshold -inf: no distance passes it, so
@@ -1083,18 +1082,13 @@ __global__ void __launch_bounds__(T)
             if constexpr (IVF) g += W;
             else g = g_lo + static_cast<int64_t>(__builtin_amdgcn_readfirstlane(grab));
         };
-        // Lane l % W holds wave l % W's value: the second smallest of the W (equal values count each).
-        auto second_smallest = [&](int v) __attribute__((always_inline)) {
-            auto smallest = [](int x) __attribute__((always_inline)) {
-                x = min(x, xor_lane<1>(x));
-                x = min(x, xor_lane<2>(x));
-                x = min(x, xor_lane<4>(x));
-                if constexpr (W > 8) x = min(x, xor_lane<8>(x));
-                return x;
-            };
-            const int low = smallest(v);
-            const int at = __ffsll(static_cast<unsigned long long>(__builtin_amdgcn_ballot_w64(v == low))) - 1;
-            return smallest(lane % W == at ? 0x7f800000 : v);
+        // Lane l % W holds wave l % W's value: the largest of the W.
+        auto largest = [&](int v) __attribute__((always_inline)) {
+            v = max(v, xor_lane<1>(v));
+            v = max(v, xor_lane<2>(v));
+            v = max(v, xor_lane<4>(v));
+            if constexpr (W > 8) v = max(v, xor_lane<8>(v));
+            return v;
         };
         // One granule step with abandoned tiles. next_heads: the granule's head codes, loaded a step ahead; dword u of
         // next_heads[h] holds codes 4h .. 4h + 3 of tile u.
@@ -1150,8 +1144,8 @@ __global__ void __launch_bounds__(T)
         // Bounds before the scan. Until a block has met vectors near a query no tile can be dropped for it, and with
         // four queries a block would sum a thousand-odd tiles in full before it has met all four's neighbourhoods. So
         // each wave first compares one vector of every tile of its share by the first kCheck sub-spaces, 64 tiles at a
-        // time, and sums the best tile of each query: the tile's K-th smallest distance is that of K real vectors (K >
-        // 64: the ceil(K/2)-th of two waves' tiles).
+        // time, and sums the best tile of each query: the tile's K-th smallest distance has K real vectors at or
+        // below it, and so has the largest of the waves' ceil(K/W)-th smallest.
         auto first_bounds = [&]() __attribute__((always_inline)) {
             float best[QS];
             uint32_t best_tile[QS];
@@ -1178,7 +1172,7 @@ __global__ void __launch_bounds__(T)
                     best_tile[q] = nearer ? tile : best_tile[q];
                 }
             }
-            const int rank = (kHalfRank && a.K > WAVE ? (a.K + 1) / 2 : a.K) - 1;
+            const int rank = a.K - 1, share = (a.K + W - 1) / W - 1;  // K <= 64
 #pragma unroll 1
             for (int i = 0; i < QS; ++i) {  // one copy of the sums and the sort
                 uint64_t key = 0;
@@ -1217,20 +1211,15 @@ __global__ void __launch_bounds__(T)
                 wave_sort<2, false>(sorted);
                 const uint32_t bound = static_cast<uint32_t>(
                     __builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(sorted >> 32)), rank));
-                if constexpr (kHalfRank) {
-                    if (a.K > WAVE) half_rank[i][wave] = static_cast<int>(bound);
-                    else atomicMin(&block_bound[i], bound);
-                } else {
-                    atomicMin(&block_bound[i], bound);
-                }
+                share_rank[i][wave] =
+                    __builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(sorted >> 32)), share);
+                if (lane == 0) atomicMin(&block_bound[i], bound);
             }
             __syncthreads();
-            if constexpr (kHalfRank) {
-                if (a.K > WAVE) {
 #pragma unroll 1
-                    for (int i = 0; i < QS; ++i)
-                        atomicMin(&block_bound[i], static_cast<unsigned>(second_smallest(half_rank[i][lane % W])));
-                }
+            for (int i = 0; i < QS; ++i) {
+                const int bound = largest(share_rank[i][lane % W]);
+                if (lane == 0) atomicMin(&block_bound[i], static_cast<unsigned>(bound));
             }
         };
         auto prune_step = [&]() __attribute__((always_inline)) {
@@ -1354,20 +1343,10 @@ __global__ void __launch_bounds__(T)
                 }
                 changed = true;
             }
-            if constexpr (kHalfRank) {
-                if (changed) {
-                    const int rank = (a.K + 1) / 2 - 1;  // < 64: in the lists' first register
-#pragma unroll
-                    for (int q = 0; q < QS; ++q) {
-                        half_rank[q][wave] = __float_as_int(lane_read(lists[q].d[0], rank));
-                        f[q] = __int_as_float(min(__float_as_int(f[q]), second_smallest(half_rank[q][lane % W])));
-                    }
-                }
-            }
             if (changed) {  // publish this wave's K-th best distances
                 int pub = 0;
 #pragma unroll
-                for (int q = 0; q < QS; ++q) pub = lane % QS == q ? __float_as_int(kHalfRank ? f[q] : lists[q].thr_d) : pub;
+                for (int q = 0; q < QS; ++q) pub = lane % QS == q ? __float_as_int(lists[q].thr_d) : pub;
                 atomicMin(&block_bound[lane % QS], static_cast<unsigned>(pub));
             }
             g = g_ahead;
@@ -1570,29 +1549,25 @@ WaveScanKernel select_wave_kernel(int qg, int ng, int ilp, int segments, bool bu
     return WaveScanKernel{};
 }
 
-// Instances that abandon tiles, for one M and entry type: one table group, four tiles per wave step, 1024-thread blocks
+// Instances that abandon tiles, for one M and entry type: one table group, lists of up to 64, four tiles per wave step, 1024-thread blocks
 // where kWideBlock holds (more waves share a bound), else 512.
 template <int M, bool F16>
-WaveScanKernel select_abandon_kernel(int q, int segments, int threads) {
+WaveScanKernel select_abandon_kernel(int q, int threads) {
     constexpr int kLds = 160 * 1024;
-#define VK_ABANDON(QG_, S_)                                                                                       \
-    if (q == QG_ && segments == S_) {                                                                            \
+#define VK_ABANDON(QG_)                                                                                           \
+    if (q == QG_) {                                                                                              \
         if constexpr (M * KSUB * Entries<QG_, F16>::kBytes <= kLds) {                                             \
-            if constexpr (kWideBlock<QG_, 1, M, S_, F16>) {                                                      \
-                if (threads == 1024) return make_wave_kernel<QG_, 1, 4, M, S_, F16, false, false, 1024, true>(); \
+            if constexpr (kWideBlock<QG_, 1, M, 1, F16>) {                                                       \
+                if (threads == 1024) return make_wave_kernel<QG_, 1, 4, M, 1, F16, false, false, 1024, true>();  \
             }                                                                                                    \
-            if (threads == 512) return make_wave_kernel<QG_, 1, 4, M, S_, F16, false, false, 512, true>();       \
+            if (threads == 512) return make_wave_kernel<QG_, 1, 4, M, 1, F16, false, false, 512, true>();        \
         }                                                                                                        \
     }
-    VK_ABANDON(1, 1)
-    VK_ABANDON(1, 2)
-    VK_ABANDON(2, 1)
-    VK_ABANDON(2, 2)
-    VK_ABANDON(4, 1)
-    VK_ABANDON(4, 2)
+    VK_ABANDON(1)
+    VK_ABANDON(2)
+    VK_ABANDON(4)
     if constexpr (F16) {
-        VK_ABANDON(8, 1)
-        VK_ABANDON(8, 2)
+        VK_ABANDON(8)
     }
 #undef VK_ABANDON
     return WaveScanKernel{};

@@ -93,9 +93,9 @@ struct WaveScanKernel {
     hipError_t (*launch)(const WaveScanArgs&, int grid, size_t smem, hipStream_t) = nullptr;
 };
 
-// The instance that abandons tiles (m = 16, 32, 48, 64; q queries in one table group; 1024 or 512 threads); fn ==
+// The instance that abandons tiles (m = 16, 32, 48, 64; q queries in one table group, K <= 64; 1024 or 512 threads); fn ==
 // nullptr when it is not built.
-WaveScanKernel abandon_kernel(int q, int m, int segments, bool f16, int threads);
+WaveScanKernel abandon_kernel(int q, int m, bool f16, int threads);
 // Returns a kernel with fn == nullptr when the combination is not built. f16: binary16 tables (v9). bulk: the
 // instance with bulk admission into one-register lists (fp32, more than one query per block only). threads: block
 // size, 512 or 1024 (built for four tiles per wave step where two 512-thread blocks' tables fit one CU).

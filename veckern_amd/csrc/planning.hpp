@@ -99,12 +99,20 @@ inline Partition balanced_partition(int64_t n, size_t nq, int q, int ilp, int64_
 // block: 11k vectors per block -26 %, 39k -11 %, 500k neutral, 5M +1 %.
 constexpr int64_t kBulkScanVectors = int64_t{1} << 18;
 
-// Vectors one block scans of one slab (the longest run of a slab's granules in one block) below the bulk limit.
-inline bool bulk_scan(const Partition& p, int ilp) {
-    if (p.grid <= 0 || p.total <= 0) return false;
-    const int64_t per_block = std::min(p.n_gran, (p.total + p.grid - 1) / p.grid);
-    return per_block * 64 * ilp < kBulkScanVectors;
+// Vectors one block scans of one slab: the longest run of a slab's granules in one block.
+inline int64_t block_vectors(const Partition& p, int ilp) {
+    if (p.grid <= 0 || p.total <= 0) return 0;
+    return std::min(p.n_gran, (p.total + p.grid - 1) / p.grid) * 64 * ilp;
 }
+inline bool bulk_scan(const Partition& p, int ilp) {
+    return p.grid > 0 && p.total > 0 && block_vectors(p, ilp) < kBulkScanVectors;
+}
+
+// Scans that abandon tiles find bounds first, which a block that scans few vectors does not earn back: at 8-10k vectors
+// per block 43 against 40 us (one query, 1M) and 59 against 58 us (100 queries, 100k), at 39k 64 against 73 us (one
+// query, 10M) and 80 against 111 us (37 queries, 1M). Lists longer than 64 do not use them either: a bound needs more
+// near vectors than a tile holds, and at k = 100 the plain scan was faster (1M, m = 16: 722 against 787 us).
+constexpr int64_t kAbandonVectors = int64_t{1} << 15;
 
 // Whether scans that abandon tiles pay: the mean squared distance between vectors of one tile (past the sort key),
 // against that between vectors far apart in the slot order. Uniform codes have a ratio of 1 and no tile can be dropped;
