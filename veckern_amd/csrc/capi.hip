@@ -1187,11 +1187,17 @@ struct vk_ivf {
         plan_ticket.ensure(1);
         if (!ticket_clean) VK_HIP(vk::launch_zero_words(plan_ticket.get(), 1, stream));
         ticket_clean = false;  // until the stream has completed this search
+        // A small search is a chain of short launches, so its tables share one with the distances; a large one fills the
+        // GPU with either, and its table blocks would hold the tiles' LDS for nothing.
+        const bool fused_tables = nq <= 64 && rows >= nq;
         clock.time(&t->lut_ms, [&] {
+            if (!fused_tables)
+                VK_HIP(vk::launch_lut(d_q, centroids.get(), static_cast<int>(d), static_cast<int>(m),
+                                      static_cast<int>(nq), 1, static_cast<int>(nq), lut.get(), stream));
             for (size_t r0 = 0; r0 < nq; r0 += rows) {
                 const size_t nr = std::min(rows, nq - r0);
-                // the tables of every query come with the first rows' distances
-                const vk::ProbeLut tables{r0 == 0 ? d_q : nullptr, centroids.get(), static_cast<int>(m),
+                // a small search's tables come with its distances
+                const vk::ProbeLut tables{fused_tables ? d_q : nullptr, centroids.get(), static_cast<int>(m),
                                           static_cast<int>(nq), lut.get()};
                 VK_HIP(vk::launch_coarse_distances(d_q + r0 * d, static_cast<int64_t>(nr), coarse.get(),
                                                    static_cast<int64_t>(nlist), static_cast<int>(d), coarse_dist.get(),
@@ -1447,6 +1453,7 @@ VK_EXPORT int vk_reranker_create(const float* base, size_t n, size_t d, vk_reran
         r->n = n;
         r->d = d;
         VK_HIP(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
+        r->error.ensure(1);
         r->base.ensure(n * d);
         VK_HIP(hipMemcpy(r->base.get(), base, n * d * sizeof(float), hipMemcpyHostToDevice));
         *out = r.release();

@@ -27,6 +27,10 @@ namespace {
 
 constexpr int kMergeThreads = 256;
 constexpr int kPlanThreads = 256;
+constexpr int kScanThreads = 1024;
+// Queries up to which the plan kernel sums the runs itself: every block then writes its XCD's L2 back before it takes
+// the ticket, which over a thousand blocks costs more than the launch it saves.
+constexpr int64_t kTicketQueries = 64;
 
 __device__ __forceinline__ int64_t wave_inclusive_sum(int64_t v) {
     const int lane = __lane_id();
@@ -38,12 +42,32 @@ __device__ __forceinline__ int64_t wave_inclusive_sum(int64_t v) {
     return v;
 }
 
+// query_gran[0..nq) from run lengths to their exclusive prefix, query_gran[nq] = total, by one block of T threads.
+template <int T>
+__device__ __forceinline__ void run_prefix(const IvfPlanArgs& a, int64_t* wave_sums) {
+    const int tid = threadIdx.x, lane = __lane_id(), wave = tid / WAVE;
+    const int64_t per = (a.nq + T - 1) / T;
+    const int64_t lo = min<int64_t>(a.nq, tid * per), hi = min<int64_t>(a.nq, lo + per);
+    int64_t sum = 0;
+    for (int64_t i = lo; i < hi; ++i) sum += a.query_gran[i];
+    const int64_t incl = wave_inclusive_sum(sum);
+    if (lane == WAVE - 1) wave_sums[wave] = incl;
+    __syncthreads();
+    int64_t run = incl - sum;
+    for (int w = 0; w < wave; ++w) run += wave_sums[w];
+    for (int64_t i = lo; i < hi; ++i) {
+        const int64_t len = a.query_gran[i];
+        a.query_gran[i] = run;
+        run += len;
+    }
+    if (tid == T - 1) a.query_gran[a.nq] = run;
+}
+
 // Probe selection and the slab plan, one block per query. Each wave streams its share of the query's coarse
 // distances into a wave list, the lists are merged by rank, and the nprobe nearest become slabs q * nprobe + p in
 // probe order: a slab's granule count is its list's padded tiles / 4 (0 for no list: a query whose coarse distances
-// are all NaN probes nothing), slab_gran receives its start within the query's run. The last block to finish (a
-// ticket, left at zero) turns the run lengths in query_gran[0..nq) into their exclusive prefix, query_gran[nq] = total.
-// One launch for what were four (row top-k, run lengths, prefix, absolute slab starts): a search of one query is a
+// are all NaN probes nothing), slab_gran receives its start within the query's run. With a ticket (left at zero), the
+// last block to finish also sums the runs; without, a launch of its own does. One launch for what were four (row top-k, run lengths, prefix, absolute slab starts): a search of one query is a
 // chain of launches that each last a few microseconds.
 template <int S>
 __global__ void __launch_bounds__(kPlanThreads) ivf_plan_kernel(IvfPlanArgs a) {
@@ -81,28 +105,23 @@ __global__ void __launch_bounds__(kPlanThreads) ivf_plan_kernel(IvfPlanArgs a) {
         }
         if (lane == 0) {
             a.query_gran[q] = run;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            last_block = atomicInc(a.ticket, static_cast<unsigned>(a.nq - 1)) == static_cast<unsigned>(a.nq - 1);
+            last_block = false;
+            if (a.ticket) {
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                last_block = atomicInc(a.ticket, static_cast<unsigned>(a.nq - 1)) == static_cast<unsigned>(a.nq - 1);
+            }
         }
     }
+    if (!a.ticket) return;
     __syncthreads();
     if (!last_block) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    const int64_t per = (a.nq + kPlanThreads - 1) / kPlanThreads;
-    const int64_t lo = min<int64_t>(a.nq, tid * per), hi = min<int64_t>(a.nq, lo + per);
-    int64_t sum = 0;
-    for (int64_t i = lo; i < hi; ++i) sum += a.query_gran[i];
-    const int64_t incl = wave_inclusive_sum(sum);
-    if (lane == WAVE - 1) wave_sums[wave] = incl;
-    __syncthreads();
-    int64_t run = incl - sum;
-    for (int w = 0; w < wave; ++w) run += wave_sums[w];
-    for (int64_t i = lo; i < hi; ++i) {
-        const int64_t len = a.query_gran[i];
-        a.query_gran[i] = run;
-        run += len;
-    }
-    if (tid == kPlanThreads - 1) a.query_gran[a.nq] = run;
+    run_prefix<kPlanThreads>(a, wave_sums);
+}
+
+__global__ void __launch_bounds__(kScanThreads) ivf_plan_prefix_kernel(IvfPlanArgs a) {
+    __shared__ int64_t wave_sums[kScanThreads / WAVE];
+    run_prefix<kScanThreads>(a, wave_sums);
 }
 
 // One wave per query streams its partial lists through a wave list (device.hpp: whole lists when long, else
@@ -135,12 +154,16 @@ __global__ void __launch_bounds__(kMergeThreads) ivf_merge_kernel(IvfMergeArgs a
 
 }  // namespace
 
-hipError_t launch_ivf_plan(const IvfPlanArgs& a, int rows, hipStream_t stream) {
-    if (a.nq <= 0 || a.nprobe <= 0 || rows <= 0) return hipErrorInvalidValue;
+hipError_t launch_ivf_plan(const IvfPlanArgs& args, int rows, hipStream_t stream) {
+    if (args.nq <= 0 || args.nprobe <= 0 || rows <= 0) return hipErrorInvalidValue;
+    IvfPlanArgs a = args;
+    if (a.nq > kTicketQueries) a.ticket = nullptr;
     const dim3 grid(static_cast<unsigned>(rows));
     if (a.K <= WAVE) hipLaunchKernelGGL(ivf_plan_kernel<1>, grid, dim3(kPlanThreads), 0, stream, a);
     else if (a.K <= 2 * WAVE) hipLaunchKernelGGL(ivf_plan_kernel<2>, grid, dim3(kPlanThreads), 0, stream, a);
     else return hipErrorInvalidValue;
+    if (!a.ticket && a.first + rows == a.nq)
+        hipLaunchKernelGGL(ivf_plan_prefix_kernel, dim3(1), dim3(kScanThreads), 0, stream, a);
     return hipGetLastError();
 }
 
