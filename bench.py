@@ -377,7 +377,8 @@ def main():
         "kernel": "fused_wave_kernel_t (scan + per-wave top-k)",
         "kernel_ms": scan_ms,
         "algorithmic": f"n*m*nq = {lookups:.3e} LDS lookups per launch (one {2 if f16 else 4}-byte table read + "
-                       f"one fp32 add each)",
+                       f"one fp32 add each), counted for every vector: scans that abandon tiles make fewer, so the "
+                       f"fraction can exceed 1",
         "peak_basis": (f"64 lookups per CU-cycle x {info.sm_count} CUs x {info.clock_khz / 1e6:.2f} GHz: the LDS "
                        f"returns 256 B/clk/CU (one 4-byte fp32 entry per lookup) and the VALU 64 lane-ops/clk/CU "
                        f"(one add, or one v_fma_mix_f32 for fp16 entries, per lookup)"),
