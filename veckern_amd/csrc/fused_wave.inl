@@ -616,6 +616,8 @@ __global__ void __launch_bounds__(T)
     // K real candidates lie at or below it, so nothing beyond it reaches the merged top K; ties at it are kept.
     // In the sorted slot order a tile's vectors are alike, so they fail together: on the 1M-vector Gaussian mixture 98 %
     // of the tiles fail for all four queries after 6 of 16 sub-spaces (65 % after 4), 90 % after 8 of 32.
+    // Measured against the plain scan: 1M x 1000 queries, m = 16, k = 10: 611 -> 308 us (fp16 tables, eight queries: 731
+    // -> 560), 37 queries 110 -> 80 us, one query over 10M 73 -> 64 us.
     // The first kHeadBytes codes of every vector are read from an array of their own (a.heads): the scan reads half of
     // the code bytes at m = 16 and a quarter at m = 32 .. 64, the rest and the ids only for tiles that are left.
     constexpr bool kPrune = ABANDON;

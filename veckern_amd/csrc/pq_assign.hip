@@ -70,7 +70,8 @@ __global__ void __launch_bounds__(kAssignThreads) nearest_kernel(NearestArgs a) 
 // the sum of their magnitudes (2^-16 X C + 2^-17 C^2 at NK = 2), the index bits 2^-17 of the value. Exact sums err by
 // at most (dsub + 3) 2^-24 of the distance, at most (X + C)^2. The gap must exceed both values' errors.
 //
-// What bounds it: the VALU work per value (at 1M x d128, m = 16: 4.1e9 values).
+// What bounds it: the VALU work per value (at 1M x d128, m = 16: 4.1e9 values; 668 us, the exact comparison of every
+// centroid took 1827).
 // Blocks of the same vectors and consecutive sub-spaces run on the same XCD (block b runs on XCD b % 8), so that a
 // 128-byte line of x, which holds several sub-spaces, is read into one L2 once.
 constexpr int kXcds = 8;

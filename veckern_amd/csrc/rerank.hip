@@ -10,7 +10,8 @@
 // The work is a random gather of r rows of d floats per query, bound by memory latency and by the addresses a CU can
 // process: a lane that reads its own row touches a line of its own with every load, 64 lines per instruction. The
 // rows therefore come in 32-float slices that consecutive lanes read together (8 lanes per 128-byte slice of a row)
-// and go through LDS to the lane that sums them, with the next slice's loads in flight meanwhile.
+// and go through LDS to the lane that sums them, with the next slice's loads in flight meanwhile (1000 queries x 100
+// candidates, d = 128: 50.8 us per call with one wave per query reading rows lane by lane, 45.7 so).
 #include <type_traits>
 
 #include "kernels.hpp"
