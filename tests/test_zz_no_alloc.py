@@ -74,6 +74,18 @@ def test_noalloc_single_query_over_many_blocks():
             assert_same(ref, new, f"nq={nq}")
 
 
+@pytest.mark.parametrize("nq,k", [(1025, 64), (1040, 64), (1500, 64), (2048, 64), (2048, 10)])
+def test_noalloc_takes_batches_of_alike_codes_that_fit_the_plain_scan(nq, k):
+    # Codes that repeat within tiles, more slabs than CUs: blocks of 1024 threads cross slab boundaries, and their
+    # partial lists (up to 2 blocks x 16 lists a query) need up to four times the scratch of 512-thread blocks, which
+    # stay aligned up to 512 slabs (8 lists a query: 512 x 4 x 8 x 64 pairs x 8 bytes = 8.4 MB, within the scratch).
+    centroids, codes, queries = datagen.pq_fixture(40_003, 64, 16, nq, seed=17)
+    with vk.PQSearcher(centroids, codes, 64) as s:
+        s.set_tuning(vk.Tuning(queries_per_block=4))
+        ref, new, _, _ = search_pair(s, queries, k, vk.ScanVariant.FusedWarp)
+        assert_same(ref, new, f"nq={nq} k={k}")
+
+
 def test_noalloc_rejects_searches_beyond_its_scratch_before_launch():
     centroids, codes, queries = datagen.random_fixture(100_003, 128, 16, 4, seed=9)
     nq, k = 20_000, 128  # 5000 slabs x 4 queries x 8 lists x 128 pairs x 8 bytes = 164 MB of partial lists

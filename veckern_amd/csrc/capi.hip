@@ -428,7 +428,8 @@ struct vk_searcher {
         size_t part_pairs = 0;  // partial-list pairs: [slabs][q][max_slots][lists_per_block][K]
     };
 
-    WavePlan plan_wave(size_t b, size_t kk, bool f16) const {
+    // may_abandon: whether the plan may take an instance that abandons tiles.
+    WavePlan plan_wave(size_t b, size_t kk, bool f16, bool may_abandon = true) const {
         WavePlan w;
         // The wave lists take any length up to 128, so they hold exactly k entries: every one of k..K-1 that a
         // rounded-up K would keep costs inserts (about K * ln(n / K) per list) and buys nothing.
@@ -452,7 +453,7 @@ struct vk_searcher {
                                                   tuning.blocks_per_query, info.sm_count);
         };
         bool abandon = false;
-        if (abandon_tiles && w.ilp == 4 && ng == 1 && segments == 1) {
+        if (may_abandon && abandon_tiles && w.ilp == 4 && ng == 1 && segments == 1) {
             vk::WaveScanKernel k;
             if (tuning.scan_threads != 512) k = vk::abandon_kernel(w.q, static_cast<int>(m), f16, 1024);
             if (!k.fn) k = vk::abandon_kernel(w.q, static_cast<int>(m), f16, 512);
@@ -759,13 +760,21 @@ struct vk_searcher {
         use_device();
         const bool f16 = v == VK_V9_FUSED_WARP_F16;
         const size_t batch = query_batch(v);
+        auto part_bytes = [](const WavePlan& w) { return w.part_pairs * sizeof(Pair); };
+        // The plan of a batch of b queries. Instances that abandon tiles keep 1024-thread blocks where the plain scan
+        // would take 512-thread ones to stay within slab boundaries, so each slab can have four times the partial
+        // lists; a search whose lists then exceed the static scratch takes the plain scan, which may fit.
+        auto plan = [&](size_t b) {
+            WavePlan w = plan_wave(b, kk, f16);
+            if (part_bytes(w) > kNoAllocScratchBytes - kNoAllocCounterBytes) w = plan_wave(b, kk, f16, false);
+            return w;
+        };
         for (size_t q0 = 0; q0 < nq; q0 += batch) {
-            const WavePlan w = plan_wave(std::min(batch, nq - q0), kk, f16);
+            const WavePlan w = plan(std::min(batch, nq - q0));
             const size_t counter_bytes = static_cast<size_t>(w.part.slabs) * sizeof(unsigned);
-            const size_t part_bytes = w.part_pairs * sizeof(Pair);
-            if (counter_bytes > kNoAllocCounterBytes || part_bytes > kNoAllocScratchBytes - kNoAllocCounterBytes)
+            if (counter_bytes > kNoAllocCounterBytes || part_bytes(w) > kNoAllocScratchBytes - kNoAllocCounterBytes)
                 fail(VK_ERR_INVALID_ARGUMENT,
-                     "vk_search_device_noalloc: this search needs " + std::to_string(part_bytes) +
+                     "vk_search_device_noalloc: this search needs " + std::to_string(part_bytes(w)) +
                          " bytes of partial lists and " + std::to_string(counter_bytes) +
                          " bytes of slab counters, beyond its static scratch (" +
                          std::to_string(kNoAllocScratchBytes - kNoAllocCounterBytes) + " and " +
@@ -789,7 +798,7 @@ struct vk_searcher {
         dev.counters_clean = false;  // until the stream has completed every launch below
         for (size_t q0 = 0; q0 < nq; q0 += batch) {
             const size_t b = std::min(batch, nq - q0);
-            const WavePlan w = plan_wave(b, kk, f16);
+            const WavePlan w = plan(b);
             // The shared bounds sit behind the counters where both fit; without them the slab's blocks scan with
             // their own bounds only (same results).
             const size_t slabs = static_cast<size_t>(w.part.slabs);
