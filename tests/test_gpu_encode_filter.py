@@ -1,7 +1,12 @@
 """GPU PQ encoding through the matrix-core filter (vk_pq_encode): codes must be the oracle's for every sub-vector width
 with an instance (2, 3, 4, 6, 8, 12, 16) and others, at sizes around a wave and a block, with near ties (centroids a few
 units in the last place apart), exact ties, magnitudes that leave the filter's range, infinities and NaN.
+Data off the origin, repeated centroids and steps that change from decided to undecided vectors must give the same
+codes, and must not fall to a slow path that costs several times the ordinary one.
 """
+import ctypes
+import time
+
 import numpy as np
 import pytest
 
@@ -47,3 +52,55 @@ def test_encode_special_values(dsub):
         c2, x2, _ = case(27 + dsub, 2_000, 3, dsub)
         c2, x2 = c2 * np.float32(scale), x2 * np.float32(scale)
         assert (vk.pq_encode(c2, x2) == orc.pq_encode(c2, x2)).all(), scale
+
+
+@pytest.mark.parametrize("dsub,m,n", [(2, 64, 70_000), (2, 3, 5_000), (3, 5, 9_001), (4, 8, 20_011), (6, 3, 4_000),
+                                      (8, 16, 9_001), (12, 4, 4_000), (16, 4, 4_000)])
+def test_encode_undecided_vectors(dsub, m, n):
+    cent, x, rng = case(41 + dsub, n, m, dsub)
+    for offset in (20.0, -1e4):  # far from the origin, where the values of one sub-vector agree in their leading digits
+        c2, x2 = cent + np.float32(offset), x + np.float32(offset)
+        assert (vk.pq_encode(c2, x2) == orc.pq_encode(c2, x2)).all(), offset
+    twice = cent.copy()
+    twice[:, 128:] = twice[:, :128]  # every vector is an exact tie
+    assert (vk.pq_encode(twice, x) == orc.pq_encode(twice, x)).all()
+    zeros = cent.copy()
+    zeros[:, 3] = zeros[:, 200] = 0.0
+    share = rng.random((n, m)) < np.linspace(0, 1, n)[:, None]  # undecided vectors: none at first, all at the end
+    x2 = x.copy()
+    x2.reshape(n, m, dsub)[share] = 0.0
+    assert (vk.pq_encode(zeros, x2) == orc.pq_encode(zeros, x2)).all()
+
+
+def device_encode_seconds(cent, x):
+    """Fastest of several device-resident encodes."""
+    n, d = x.shape
+    dc, dx, dcodes = vk.DeviceArray.from_host(cent), vk.DeviceArray.from_host(x), vk.DeviceArray(n * cent.shape[0])
+    best = np.inf
+    try:
+        for _ in range(8):
+            t = time.perf_counter()
+            rc = vk.library().vk_pq_encode_device(ctypes.c_void_p(dc.address), d, cent.shape[0],
+                                                  ctypes.c_void_p(dx.address), n, ctypes.c_void_p(dcodes.address))
+            best = min(best, time.perf_counter() - t)
+            assert rc == vk.VK_OK
+    finally:
+        dc.free()
+        dx.free()
+        dcodes.free()
+    return best
+
+
+@pytest.mark.parametrize("dsub,m", [(2, 64), (4, 32), (8, 16)])
+def test_encode_time_does_not_hang_on_the_data(dsub, m):
+    cent, x, _ = case(61, 200_000, m, dsub)
+    plain = device_encode_seconds(cent, x)
+    moved = device_encode_seconds(cent + np.float32(100), x + np.float32(100))
+    twice = cent.copy()
+    twice[:, 128:] = twice[:, :128]
+    ties = device_encode_seconds(twice, x)
+    # Moved data is decided like the rest; exact ties cost one exact comparison of every centroid, 9 / 3, 15 / 3 and
+    # 27 / 3 VALU operations per value at most against the filter's (1.1, 1.8 and 2.6 times its time measured; all of
+    # them one after another were 3.3, 3.8 and 4.6 times).
+    assert moved < 1.5 * plain, (plain, moved)
+    assert ties < {2: 2.0, 4: 2.6, 8: 3.6}[dsub] * plain, (plain, ties)
