@@ -144,6 +144,21 @@ int vk_searcher_last_launch(const vk_searcher* s, vk_launch_shape* out);
  * (VK_ERR_INVALID_ARGUMENT). */
 int vk_searcher_layout(vk_searcher* s, uint32_t* ids, size_t ids_count, uint8_t* rows, size_t rows_count, int* lanes);
 
+/* Tile abandonment of the v8/v9 scans: a 64-vector tile is dropped when its partial sums exceed every query's bound
+ * (identical results). AUTO (the default) uses it where the layout found the codes of a tile alike and a block scans
+ * enough vectors; ALWAYS wherever an instance exists (m = 16, 32, 48 or 64, k <= 64, four tiles per step, fp32 tables of
+ * up to 4 queries or fp16 tables of up to 8); NEVER nowhere. No counterpart in the reference; for tests and
+ * measurements. */
+enum vk_abandon { VK_ABANDON_AUTO = 0, VK_ABANDON_ALWAYS = 1, VK_ABANDON_NEVER = 2 };
+int vk_searcher_set_abandon(vk_searcher* s, int mode);
+/* The kernel instance of the last v8/v9 scan: queries per table, tables per block, 64-vector tiles per wave step,
+ * compile-time sub-spaces (0: any m), list registers per lane, threads per block, fp16 tables, bulk admission, tile
+ * abandonment. VK_ERR_LOGIC before the first such search. No counterpart in the reference; for tests and tools. */
+typedef struct vk_scan_kernel {
+    int queries_per_table, tables, tiles_per_step, sub_spaces, list_registers, threads, f16, bulk, abandons;
+} vk_scan_kernel;
+int vk_searcher_last_kernel(const vk_searcher* s, vk_scan_kernel* out);
+
 /* gpu.hpp:61 search (searcher.cu:466-520): out[nq * k] host memory, ascending (dist, id) per query, padded
  * {+inf, -1}. Errors: k not in [1, min(128, n)] (VK_ERR_RUNTIME), m % 16 != 0 for v2/v6/v7/v8 or tables that
  * do not fit in LDS (VK_ERR_RUNTIME). timings may be NULL. nq == 0 is a no-op. */

@@ -1,8 +1,11 @@
 """GPU fused scan with abandoned tiles: a 64-vector tile is dropped when its partial sums after a quarter or half of the
 sub-spaces already exceed every query's admission bound, the bounds shared between the waves of a block and the blocks
 of a slab. Results must stay those of the oracle, bit for bit, for clustered codes (most tiles dropped), uniform codes
-(hardly any), exact ties at the bound, distances that overflow to infinity, padded query slots, and repeated searches
-of one searcher with changing shapes (the shared bounds return to their initial state).
+(hardly any), exact ties at the bound, distances that overflow to infinity, NaN, padded query slots, and repeated
+searches of one searcher with changing shapes (the shared bounds return to their initial state).
+
+Left to itself a searcher abandons tiles only where its codes are alike within tiles and a block scans many vectors, so
+the families run with abandonment forced as well, and the kernel that ran is asserted.
 """
 import numpy as np
 import pytest
@@ -28,9 +31,27 @@ def fixture(family, n, d, m, nq):
         return datagen.random_fixture(n, d, m, nq, seed=901 + m)
     if family == "ties":
         return datagen.tie_fixture(n, d, m, nq, seed=902 + m)
+    if family == "clustered ties":  # few distinct vectors, in clusters: whole tiles tie with the K-th best
+        rng = np.random.default_rng(904 + m)
+        cent = rng.integers(0, 3, size=(m, 256, d // m)).astype(np.float32)
+        kinds = rng.integers(0, 256, size=(300, m), dtype=np.uint8)
+        queries = rng.integers(0, 3, size=(nq, d)).astype(np.float32)
+        return cent, kinds[rng.integers(0, 300, n)], queries
     cent, codes, queries = datagen.pq_fixture(n, d, m, nq, seed=903 + m)
+    if family == "nan":
+        cent[3, 40:90, 0] = np.nan  # NaN distances among finite ones
+        queries[1] = np.nan         # and a query that has no other
+        queries[4, 2] = np.inf
+        return cent, codes, queries
     cent[:, 5:60] *= np.float32(1e19)  # squares overflow: infinite distances among finite ones
     return cent, codes, queries
+
+
+def expect_abandoned(s, k, q):
+    """The last scan abandoned tiles exactly where an instance exists."""
+    kernel = s.last_kernel()
+    assert kernel.abandons == (k <= 64 and kernel.tables == 1), kernel
+    assert kernel.queries_per_table * kernel.tables <= q
 
 
 @pytest.mark.parametrize("family", ["clusters", "uniform", "ties", "overflow"])
@@ -49,13 +70,61 @@ def test_abandoned_tiles_match_oracle(family, d, m):
             assert_same(got_d, got_i, orc.adc_search_f16(cent, d, codes, queries, 10), f"v9 Q={q} threads={threads}")
 
 
+@pytest.mark.parametrize("family", ["clusters", "uniform", "ties", "clustered ties", "overflow", "nan"])
+@pytest.mark.parametrize("d,m", [(64, 16), (64, 32), (96, 48), (128, 64)])
+def test_forced_abandonment_matches_oracle(family, d, m):
+    n, nq = 20_003, 21
+    cent, codes, queries = fixture(family, n, d, m, nq)
+    with np.errstate(all="ignore"), vk.PQSearcher(cent, codes, d) as s:
+
+        def expected(count, k, variant):
+            if family == "nan":  # the order of NaN distances is not defined: as the plain scan has it
+                s.set_abandon(vk.Abandon.Never)
+                dist, ids, _ = s.search(queries[:count], k, variant)
+                assert not s.last_kernel().abandons
+                s.set_abandon(vk.Abandon.Always)
+                exp = np.empty(ids.shape, dtype=vk.NEIGHBOR_DTYPE)
+                exp["dist"], exp["id"] = dist, ids
+                return exp
+            return (orc.adc_search if variant == V8 else orc.adc_search_f16)(cent, d, codes, queries[:count], k)
+
+        s.set_abandon(vk.Abandon.Always)
+        for q, threads, blocks in [(1, 256, 4), (2, 1024, 2), (4, 512, 1), (4, 1024, 7), (4, 256, 0), (8, 256, 3)]:
+            s.set_tuning(vk.Tuning(queries_per_block=q, scan_threads=threads, blocks_per_query=blocks))
+            for variant, k, count in [(V8, 1, nq), (V8, 10, 1), (V8, 16, nq), (V8, 64, 5), (V8, 65, nq), (V9, 10, nq)]:
+                got_d, got_i, _ = s.search(queries[:count], k, variant)
+                expect_abandoned(s, k, q)
+                assert_same(got_d, got_i, expected(count, k, variant),
+                            f"{vk.variant_name(variant)} Q={q} threads={threads} blocks={blocks} k={k} nq={count}")
+
+
+def test_abandonment_modes():
+    cent, codes, queries = datagen.pq_fixture(140_003, 64, 16, 4, seed=930)
+    exp = orc.adc_search(cent, 64, codes, queries, 10)
+    with vk.PQSearcher(cent, codes, 64) as s:
+        with pytest.raises(vk.VkLogicError):
+            s.last_kernel()
+        with pytest.raises(vk.VkInvalidArgument):
+            s.set_abandon(3)
+        for blocks, mode, abandons in [(1, vk.Abandon.Auto, True), (16, vk.Abandon.Auto, False),
+                                       (16, vk.Abandon.Always, True), (1, vk.Abandon.Never, False)]:
+            s.set_abandon(mode)
+            s.set_tuning(vk.Tuning(queries_per_block=4, blocks_per_query=blocks))
+            got_d, got_i, _ = s.search(queries, 10, V8)
+            assert s.last_kernel().abandons == abandons, (blocks, mode)
+            assert_same(got_d, got_i, exp, f"blocks={blocks} mode={mode}")
+
+
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 4097])
 def test_abandoned_tiles_small_databases(n):
     cent, codes, queries = datagen.random_fixture(n, 64, 16, 5, seed=910 + n)
     with vk.PQSearcher(cent, codes, 64) as s:
-        for k in (1, min(n, 100)):
-            got_d, got_i, _ = s.search(queries, k, V8)
-            assert_same(got_d, got_i, orc.adc_search(cent, 64, codes, queries, k), f"n={n} k={k}")
+        for mode in (vk.Abandon.Auto, vk.Abandon.Always):
+            s.set_abandon(mode)
+            for k in sorted({1, min(n, 60), min(n, 100)}):
+                got_d, got_i, _ = s.search(queries, k, V8)
+                assert s.last_kernel().abandons == (mode == vk.Abandon.Always and k <= 64)
+                assert_same(got_d, got_i, orc.adc_search(cent, 64, codes, queries, k), f"n={n} k={k}")
 
 
 def test_single_query_over_many_blocks_repeats():
@@ -67,5 +136,7 @@ def test_single_query_over_many_blocks_repeats():
             q = r % 4
             got_d, got_i, _ = s.search(queries[q:q + 1], 10, V8)
             assert_same(got_d, got_i, exp[q:q + 1], f"repeat {r}")
+            assert s.last_kernel().abandons
             got_d, got_i, _ = s.search(queries, 10, V8)
+            assert s.last_kernel().abandons
             assert_same(got_d, got_i, exp, f"batch {r}")

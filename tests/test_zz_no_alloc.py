@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import veckern_amd as vk
+from oracle import binding as orc
 from tests import datagen
 
 pytestmark = pytest.mark.gpu
@@ -72,6 +73,26 @@ def test_noalloc_single_query_over_many_blocks():
         for nq in (3, 1):
             ref, new, _, _ = search_pair(s, queries[:nq], 10, vk.ScanVariant.FusedWarp)
             assert_same(ref, new, f"nq={nq}")
+
+
+@pytest.mark.parametrize("variant,q", [(vk.ScanVariant.FusedWarp, 4), (vk.ScanVariant.FusedWarp, 1),
+                                       (vk.ScanVariant.FusedWarpF16, 8)])
+def test_noalloc_abandoned_tiles(variant, q):
+    # Searches that share bounds between blocks, with different numbers of slabs in turn: the bounds lie behind the slab
+    # counters in the static scratch and must be back at zero for the next search, which counts there.
+    centroids, codes, queries = datagen.pq_fixture(6_003, 64, 16, 9_000, seed=23)
+    with vk.PQSearcher(centroids, codes, 64) as s:
+        s.set_abandon(vk.Abandon.Always)
+        for nq, blocks in [(30, 5), (3, 8), (700, 2), (1, 8), (60, 3), (9_000, 2), (30, 5)]:
+            # 9000 queries, one per slab: the counters fill more than half of their part of the scratch, no bounds
+            k = 1 if nq == 9_000 else 10
+            s.set_tuning(vk.Tuning(queries_per_block=q, blocks_per_query=blocks))
+            ref, new, _, _ = search_pair(s, queries[:nq], k, variant)
+            assert s.last_kernel().abandons
+            assert_same(ref, new, f"nq={nq} blocks={blocks}")
+            expected = (orc.adc_search_f16 if variant == vk.ScanVariant.FusedWarpF16 else orc.adc_search)(
+                centroids, 64, codes, queries[:nq], k)
+            assert_same(expected, new, f"oracle nq={nq} blocks={blocks}")
 
 
 @pytest.mark.parametrize("nq,k", [(1025, 64), (1040, 64), (1500, 64), (2048, 64), (2048, 10)])

@@ -78,6 +78,12 @@ class _LaunchShape(ctypes.Structure):
                 ("blocks_per_sm", ctypes.c_int), ("waves", ctypes.c_double)]
 
 
+class _ScanKernel(ctypes.Structure):
+    _fields_ = [("queries_per_table", ctypes.c_int), ("tables", ctypes.c_int), ("tiles_per_step", ctypes.c_int),
+                ("sub_spaces", ctypes.c_int), ("list_registers", ctypes.c_int), ("threads", ctypes.c_int),
+                ("f16", ctypes.c_int), ("bulk", ctypes.c_int), ("abandons", ctypes.c_int)]
+
+
 class _DeviceInfo(ctypes.Structure):
     _fields_ = [("name", ctypes.c_char * 256), ("arch", ctypes.c_char * 64), ("sm_count", ctypes.c_int),
                 ("peak_bandwidth_gbs", ctypes.c_double), ("max_smem_per_block", ctypes.c_size_t),
@@ -106,6 +112,8 @@ _SIGNATURES = {
     "vk_searcher_set_tuning": (ctypes.c_int, [_P, ctypes.POINTER(_Tuning)]),
     "vk_searcher_get_tuning": (ctypes.c_int, [_P, ctypes.POINTER(_Tuning)]),
     "vk_searcher_last_launch": (ctypes.c_int, [_P, ctypes.POINTER(_LaunchShape)]),
+    "vk_searcher_set_abandon": (ctypes.c_int, [_P, ctypes.c_int]),
+    "vk_searcher_last_kernel": (ctypes.c_int, [_P, ctypes.POINTER(_ScanKernel)]),
     "vk_searcher_layout": (ctypes.c_int, [_P, _P, ctypes.c_size_t, _P, ctypes.c_size_t, _P]),
     "vk_search": (ctypes.c_int, [_P, _P, ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int, _P,
                                  ctypes.POINTER(_Timings)]),
@@ -204,6 +212,37 @@ class LaunchShape:
     vectors_per_step: int = 1
     blocks_per_sm: int = 0
     waves: float = 0.0
+
+
+class Abandon(enum.IntEnum):
+    """Tile abandonment of the v8/v9 scans (vk_abandon): same results, for tests and measurements."""
+
+    Auto = 0
+    Always = 1
+    Never = 2
+
+
+@dataclass
+class ScanKernel:
+    """The kernel instance of a v8/v9 scan (vk_scan_kernel)."""
+
+    queries_per_table: int
+    tables: int
+    tiles_per_step: int
+    sub_spaces: int
+    list_registers: int
+    threads: int
+    f16: bool
+    bulk: bool
+    abandons: bool
+
+    @property
+    def symbol(self) -> str:
+        """The kernel's name as a profiler prints it."""
+        numbers = (self.queries_per_table, self.tables, self.tiles_per_step, self.sub_spaces, self.list_registers,
+                   self.threads)
+        flags = (self.f16, False, self.bulk, self.abandons)
+        return f"fused_wave_kernel_t<{', '.join([str(n) for n in numbers] + [str(f).lower() for f in flags])}>"
 
 
 @dataclass
@@ -328,6 +367,15 @@ class PQSearcher:
         _check(library().vk_searcher_last_launch(self._h, ctypes.byref(s)))
         return LaunchShape(s.threads, s.blocks_x, s.grid_y, s.queries_per_block, s.vectors_per_step,
                            s.blocks_per_sm, s.waves)
+
+    def set_abandon(self, mode: int) -> None:
+        _check(library().vk_searcher_set_abandon(self._h, int(mode)))
+
+    def last_kernel(self) -> ScanKernel:
+        k = _ScanKernel()
+        _check(library().vk_searcher_last_kernel(self._h, ctypes.byref(k)))
+        return ScanKernel(k.queries_per_table, k.tables, k.tiles_per_step, k.sub_spaces, k.list_registers, k.threads,
+                          bool(k.f16), bool(k.bulk), bool(k.abandons))
 
     def search(self, queries: np.ndarray, k: int, variant: int = ScanVariant.FusedWarp):
         """Returns (dist [nq, k] float32, ids [nq, k] int32, Timings)."""

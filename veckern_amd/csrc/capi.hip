@@ -278,8 +278,11 @@ struct vk_searcher {
     hipStream_t stream = nullptr;
     DeviceBuffer<float> centroids, queries, lut, dists;
     DeviceBuffer<uint8_t> codes, codes_il;
-    DeviceBuffer<uint4> heads;             // the first codes of the sorted layout (abandon_tiles)
-    bool abandon_tiles = false;            // the codes repeat within tiles: scans with abandoned tiles
+    DeviceBuffer<uint4> heads;             // the first codes of the sorted layout, for scans that abandon tiles
+    bool have_heads = false;
+    bool codes_alike = false;              // the codes repeat within tiles (choose_abandon)
+    int abandon_mode = VK_ABANDON_AUTO;
+    vk_scan_kernel last_kernel{};          // threads = 0 before the first v8/v9 scan
     DeviceBuffer<uint4> codes_v, codes_s;  // words in vector order (v6, v7) and in sorted slot order (v8, v9)
     DeviceBuffer<uint32_t> slot_ids;        // the sorted slot order: the vector id of each slot (m % 16 == 0 only)
     DeviceBuffer<uint8_t> table_rows;       // [m][256]: the LDS table row of each code value in the sorted layout
@@ -328,6 +331,13 @@ struct vk_searcher {
             choose_abandon();
             have_s = built = true;
         }
+        if (vk::plan::uses_sorted_layout(v) && !have_heads && m <= 64 &&
+            (abandon_mode == VK_ABANDON_ALWAYS || (abandon_mode == VK_ABANDON_AUTO && codes_alike))) {
+            const int words = vk::abandon_head_words(static_cast<int>(m));
+            heads.ensure(static_cast<size_t>(n_pad / 256) * words * vk::WAVE);
+            VK_HIP(vk::launch_build_heads(codes_s.get(), static_cast<int>(m), n_pad, words, heads.get(), stream));
+            have_heads = built = true;
+        }
         if (built) VK_HIP(hipStreamSynchronize(stream));  // a layout kernel's failure surfaces here, not mid-search
     }
 
@@ -345,11 +355,7 @@ struct vk_searcher {
         double sums[2] = {0.0, 0.0};
         VK_HIP(hipMemcpyAsync(sums, spread.get(), sizeof sums, hipMemcpyDeviceToHost, stream));
         VK_HIP(hipStreamSynchronize(stream));
-        abandon_tiles = vk::plan::abandon_pays(sums[0], sums[1]);
-        if (!abandon_tiles) return;
-        const int words = vk::abandon_head_words(static_cast<int>(m));
-        heads.ensure(static_cast<size_t>(n_pad / 256) * words * vk::WAVE);
-        VK_HIP(vk::launch_build_heads(codes_s.get(), static_cast<int>(m), n_pad, words, heads.get(), stream));
+        codes_alike = vk::plan::abandon_pays(sums[0], sums[1]);
     }
 
     // The slot order and table rows of the fused scans' layout (slot_order.hpp), for table reads of `lanes` lanes
@@ -425,6 +431,7 @@ struct vk_searcher {
         size_t smem = 0;
         int q = 1, ilp = 1, K = 0, per_cu = 1, lists_per_block = 1;
         vk::plan::Partition part;
+        vk_scan_kernel id{};    // the instance
         size_t part_pairs = 0;  // partial-list pairs: [slabs][q][max_slots][lists_per_block][K]
     };
 
@@ -452,15 +459,17 @@ struct vk_searcher {
                                                   static_cast<int64_t>(w.per_cu) * info.sm_count,
                                                   tuning.blocks_per_query, info.sm_count);
         };
-        bool abandon = false;
-        if (may_abandon && abandon_tiles && w.ilp == 4 && ng == 1 && segments == 1) {
+        bool abandon = false, bulk_lists = false;
+        const bool always = abandon_mode == VK_ABANDON_ALWAYS;
+        if (may_abandon && have_heads && (always || (codes_alike && abandon_mode == VK_ABANDON_AUTO)) && w.ilp == 4 &&
+            ng == 1 && segments == 1) {
             vk::WaveScanKernel k;
             if (tuning.scan_threads != 512) k = vk::abandon_kernel(w.q, static_cast<int>(m), f16, 1024);
             if (!k.fn) k = vk::abandon_kernel(w.q, static_cast<int>(m), f16, 512);
             if (k.fn) {
                 w.kern = k;
                 plan_for(w.kern);
-                abandon = vk::plan::block_vectors(w.part, w.ilp) >= vk::plan::kAbandonVectors;
+                abandon = always || vk::plan::block_vectors(w.part, w.ilp) >= vk::plan::kAbandonVectors;
             }
         }
         if (!abandon) w.kern = vk::fused_wave_kernel(qg, ng, w.ilp, static_cast<int>(m), segments, f16);
@@ -498,8 +507,13 @@ struct vk_searcher {
                                                static_cast<int>(w.smem)));
                 VK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&bulk_per_cu, bulk.fn, bulk.threads, w.smem));
             }
-            if (bulk.fn && std::max(bulk_per_cu, 1) == w.per_cu) w.kern = bulk;
+            if (bulk.fn && std::max(bulk_per_cu, 1) == w.per_cu) {
+                w.kern = bulk;
+                bulk_lists = true;
+            }
         }
+        w.id = vk_scan_kernel{qg, ng, w.ilp, w.kern.dynamic_lds ? 0 : static_cast<int>(m), segments, w.kern.threads,
+                              f16, bulk_lists, abandon};
         // Up to 8 blocks per slab every wave leaves its own partial lists; beyond that the block merges its wave
         // lists first, which keeps the final merge of a slab to at most max(64, blocks per slab) lists per query.
         w.lists_per_block = w.part.max_slots > 8 ? 1 : w.kern.threads / vk::WAVE;
@@ -519,6 +533,8 @@ struct vk_searcher {
         last.vectors_per_step = w.ilp;
         last.blocks_per_sm = w.per_cu;
         last.waves = static_cast<double>(w.part.grid) / (static_cast<double>(w.per_cu) * info.sm_count);
+
+        last_kernel = w.id;
 
         // One launch: every block builds its slab's tables in LDS, scans, and the last block of each slab merges
         // the slab's partial lists into d_out.
@@ -1005,6 +1021,23 @@ VK_EXPORT int vk_searcher_last_launch(const vk_searcher* s, vk_launch_shape* out
     return guarded([&] {
         require(s != nullptr && out != nullptr, "null argument");
         *out = s->last;
+    });
+}
+
+VK_EXPORT int vk_searcher_set_abandon(vk_searcher* s, int mode) {
+    return guarded([&] {
+        require(s != nullptr, "searcher must not be null");
+        if (mode < VK_ABANDON_AUTO || mode > VK_ABANDON_NEVER)
+            fail(VK_ERR_INVALID_ARGUMENT, "unknown abandonment mode " + std::to_string(mode));
+        s->abandon_mode = mode;
+    });
+}
+
+VK_EXPORT int vk_searcher_last_kernel(const vk_searcher* s, vk_scan_kernel* out) {
+    return guarded([&] {
+        require(s != nullptr && out != nullptr, "searcher and out must not be null");
+        if (s->last_kernel.threads == 0) fail(VK_ERR_LOGIC, "no v8 or v9 search yet");
+        *out = s->last_kernel;
     });
 }
 
