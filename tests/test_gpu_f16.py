@@ -98,14 +98,17 @@ def test_f16_other_m_and_tie_heavy_data(family, m):
                 assert_same(got_d, got_i, exp, f"{family} m={m} Q={q} k={k}")
 
 
-def test_f16_generic_m_path():
-    n, d, m, nq = 9_001, 96, 48, 9
+@pytest.mark.parametrize("d,m", [(96, 48), (160, 80), (224, 112)])
+def test_f16_generic_m_path(d, m):
+    n, nq = 9_001, 9
     centroids, codes, queries = datagen.random_fixture(n, d, m, nq, seed=4)
     with vk.PQSearcher(centroids, codes, d) as s:
-        for q in (1, 2, 4):
+        for q in (1, 2, 4) if m == 48 else (1, 2):
             s.set_tuning(vk.Tuning(queries_per_block=q))
             got_d, got_i, _ = s.search(queries, 10, F16)
-            assert_same(got_d, got_i, orc.adc_search_f16(centroids, d, codes, queries, 10), f"m=48 Q={q}")
+            assert_same(got_d, got_i, orc.adc_search_f16(centroids, d, codes, queries, 10), f"m={m} Q={q}")
+            kernel = s.last_kernel()
+            assert (kernel.sub_spaces, kernel.queries_per_table, kernel.f16) == (48 if m == 48 else 0, q, True)
 
 
 @pytest.mark.parametrize("scale", [300.0, 1e-3])

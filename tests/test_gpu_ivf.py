@@ -103,13 +103,15 @@ def test_ivf_other_m_and_ties(family, m):
                         f"{family} m={m} nprobe={nprobe} k={k}")
 
 
-def test_ivf_generic_m_and_tiny_lists():
-    coarse, cent, codes, list_ids, queries = ivf_case(95, 3_001, 96, 48, 9, 500)  # ~6 vectors per list
+@pytest.mark.parametrize("dim,m", [(96, 48), (160, 80), (224, 112)])  # the last two have no instance of their own
+def test_ivf_generic_m_and_tiny_lists(dim, m):
+    coarse, cent, codes, list_ids, queries = ivf_case(95, 3_001, dim, m, 9, 500)  # ~6 vectors per list
     with vk.IVFIndex(coarse, cent, codes, list_ids) as ix:
         for nprobe in (1, 5, 128):
-            d, i, _ = ix.search(queries, nprobe, 10)
-            assert_same(d, i, orc.ivf_search(coarse, cent, 96, codes, list_ids, queries, nprobe, 10),
-                        f"m=48 nprobe={nprobe}")
+            for k in (10, 100):
+                d, i, _ = ix.search(queries, nprobe, k)
+                assert_same(d, i, orc.ivf_search(coarse, cent, dim, codes, list_ids, queries, nprobe, k),
+                            f"m={m} nprobe={nprobe} k={k}")
 
 
 def test_ivf_rejects_bad_arguments(index_case):

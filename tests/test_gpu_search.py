@@ -229,15 +229,18 @@ def test_admission_bursts_from_falling_distances():
                 assert_same(got_d, got_i, exp, f"falling k={k} Q={q}")
 
 
-def test_generic_m_path():
-    # m = 48 is not one of the compile-time specialisations; the kernel reads m at run time.
-    n, d, m, nq = 9_001, 96, 48, 9
+@pytest.mark.parametrize("d,m", [(96, 48), (160, 80), (224, 112)])
+def test_generic_m_path(d, m):
+    # m = 80 and 112 are not among the compile-time specialisations (48 is): the kernel reads m at run time.
+    n, nq = 9_001, 9
     centroids, codes, queries = datagen.random_fixture(n, d, m, nq, seed=3)
     with vk.PQSearcher(centroids, codes, d) as s:
-        for q in (1, 2):
+        for q in (1, 2) if m == 48 else (1,):
             s.set_tuning(vk.Tuning(queries_per_block=q))
-            got_d, got_i, _ = s.search(queries, 10, vk.ScanVariant.FusedWarp)
-            assert_same(got_d, got_i, orc.adc_search(centroids, d, codes, queries, 10), f"m=48 Q={q}")
+            for k in (10, 100):
+                got_d, got_i, _ = s.search(queries, k, vk.ScanVariant.FusedWarp)
+                assert_same(got_d, got_i, orc.adc_search(centroids, d, codes, queries, k), f"m={m} Q={q} k={k}")
+                assert s.last_kernel().sub_spaces == (48 if m == 48 else 0)
 
 
 def test_tiny_database_and_k_equal_n():
