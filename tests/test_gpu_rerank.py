@@ -56,6 +56,38 @@ def test_rerank_other_dims_and_ties(d, family):
             assert_same(got_d, got_i, orc.rerank_exact(base, queries, cand, k), f"d={d} {family} k={k}")
 
 
+# Rows read by their own lane, or slices of 64 rows: from 513 candidates (65 for d <= 32) where d % 16 == 0, and for long
+# rows from 2^24 gathered values (384 x 65 x 672).
+@pytest.mark.parametrize("d,r,nq", [(16, 64, 9), (16, 65, 9), (32, 200, 9), (48, 65, 9), (48, 512, 5), (48, 513, 5),
+                                    (100, 700, 5), (130, 700, 5), (200, 1025, 5), (384, 65, 671), (384, 65, 672),
+                                    (400, 600, 71), (960, 10, 40), (960, 300, 59)])
+def test_rerank_ways_to_read_rows(d, r, nq):
+    base, queries, cand = case(65 + d + r, 2_000, d, nq, r)
+    with vk.Reranker(base) as rr:
+        for k in (10, 100):
+            got_d, got_i, _ = rr.rerank(queries, cand, k)
+            assert_same(got_d, got_i, orc.rerank_exact(base, queries, cand, k), f"d={d} r={r} nq={nq} k={k}")
+
+
+def test_rerank_time_of_few_long_rows():
+    # The same bytes as 10 rows of 960 and as 75 rows of 128 values per query: few long rows must not be read with little
+    # in flight (1.2 times the time measured; 2.9 times when 64 rows' slices held the 10).
+    seconds = {}
+    for d, r in ((960, 10), (128, 75)):
+        base, queries, cand = case(90, 50_000, d, 2_000, r)
+        dq, dc = vk.DeviceArray.from_host(queries), vk.DeviceArray.from_host(cand)
+        dout = vk.DeviceArray(2_000 * 10 * vk.NEIGHBOR_DTYPE.itemsize)
+        try:
+            with vk.Reranker(base) as rr:
+                seconds[d] = min(rr.rerank_device(dq.address, 2_000, dc.address, r, 10, dout.address).scan_ms
+                                 for _ in range(30))
+        finally:
+            dq.free()
+            dc.free()
+            dout.free()
+    assert seconds[960] < 1.7 * seconds[128], seconds
+
+
 def test_rerank_all_padding_and_empty_batch():
     base, queries, cand = case(70, 1_000, 64, 5, 40)
     cand["id"][:] = -1

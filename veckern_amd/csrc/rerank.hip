@@ -8,10 +8,16 @@
 // The wave lists are merged through LDS.
 //
 // The work is a random gather of r rows of d floats per query, bound by memory latency and by the addresses a CU can
-// process: a lane that reads its own row touches a line of its own with every load, 64 lines per instruction. The
-// rows therefore come in 32-float slices that consecutive lanes read together (8 lanes per 128-byte slice of a row)
-// and go through LDS to the lane that sums them, with the next slice's loads in flight meanwhile (1000 queries x 100
-// candidates, d = 128: 50.8 us per call with one wave per query reading rows lane by lane, 45.7 so).
+// process. Two ways to read the rows, chosen by launch_rerank:
+//  - rows: a lane reads its own row with 16-byte loads, eight in flight;
+//  - slices: 32 floats of 64 rows at a time, 8 consecutive lanes on a 128-byte slice of a row, through LDS to the lane that
+//    sums them, with the next slice's loads in flight meanwhile. A lane that reads its own row touches a line of its own
+//    with every load, 64 lines per instruction, which costs where many rows are read per wave; a slice costs a pass through
+//    LDS each, 30 in a row for d = 960, and twice the lines where rows are not whole lines.
+// us per call, rows / slices: d = 128, 2000 x 100 34.6 / 35.8, 300 x 1000 56.2 / 45.5, one query x 100 19.0 / 21.4; d = 200,
+// 2000 x 100 47.0 / 53.0; d = 130, 2000 x 100 54.6 / 72.1; d = 384, 1000 x 1000 297 / 244; d = 960, 2000 x 10 37.1 / 65.8,
+// 1000 x 200 147 / 131, one query x 100 28.8 / 49.7; d = 16, 1000 x 1000 57.7 / 40.2. One wave per query reading rows lane
+// by lane: d = 128, 2000 x 100 54, 300 x 1000 101.
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -24,38 +30,29 @@ constexpr int kSliceFloats = 32;
 constexpr int kMaxRerankWaves = 8;
 constexpr int kSliceBytes = WAVE * kSliceFloats * 4;  // LDS per wave
 
-// One wave's slices of its 64 rows. VEC4: 16-byte loads (d % 4 == 0: rows are 16-byte aligned); otherwise 4-byte.
+// One wave's slices of its 64 rows (d % 4 == 0 and an aligned base: 16-byte loads).
 // LDS holds row-major 16-byte chunks, chunk c of row r at r * 8 + (c ^ ((r >> 1) & 7)): the 16 lanes that read the
 // same chunk of 16 consecutive rows in one pass then fall on all 16 bank groups.
-template <bool VEC4>
 struct SliceLoader {
-    static constexpr int kLoads = VEC4 ? 8 : 32;
-    using T = std::conditional_t<VEC4, float4, float>;
-    T v[kLoads];
+    static constexpr int kLoads = 8, kLanesPerRow = 8, kRows = WAVE / kLanesPerRow;
+    float4 v[kLoads];
 
     __device__ __forceinline__ void load(const float* base, int d, int32_t id, bool use, int first, int lane) {
-        constexpr int kLanesPerRow = VEC4 ? 8 : 32, kRows = WAVE / kLanesPerRow, kWidth = VEC4 ? 4 : 1;
-        const int at = first + (lane % kLanesPerRow) * kWidth;
+        const int at = first + lane % kLanesPerRow * 4;
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
-            const int row = i * kRows + lane / kLanesPerRow;
-            const int32_t rid = __shfl(use ? id : -1, row);
-            T x{};
-            if (rid >= 0 && at < d) x = *reinterpret_cast<const T*>(base + static_cast<int64_t>(rid) * d + at);
+            const int32_t rid = __shfl(use ? id : -1, i * kRows + lane / kLanesPerRow);
+            float4 x{};
+            if (rid >= 0 && at < d) x = *reinterpret_cast<const float4*>(base + static_cast<int64_t>(rid) * d + at);
             v[i] = x;
         }
     }
     __device__ __forceinline__ void store(float* lds, int lane) const {
-        constexpr int kLanesPerRow = VEC4 ? 8 : 32, kRows = WAVE / kLanesPerRow;
         const int c = lane % kLanesPerRow;
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             const int row = i * kRows + lane / kLanesPerRow;
-            if constexpr (VEC4) {
-                *reinterpret_cast<float4*>(lds + (row * 8 + (c ^ ((row >> 1) & 7))) * 4) = v[i];
-            } else {
-                lds[(row * 8 + ((c >> 2) ^ ((row >> 1) & 7))) * 4 + (c & 3)] = v[i];
-            }
+            *reinterpret_cast<float4*>(lds + (row * 8 + (c ^ ((row >> 1) & 7))) * 4) = v[i];
         }
     }
 };
@@ -66,7 +63,34 @@ __device__ __forceinline__ void wave_lds_fence() {  // LDS written by other lane
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int S, bool VEC4>
+// The distance of one candidate by its own lane, which reads the row with loads of its own, eight in flight.
+template <bool VEC4>
+__device__ __forceinline__ float row_distance(const float* x, const float* row, int d) {
+#pragma clang fp contract(off)
+    float acc = 0.f;
+    auto add = [&](float xv, float bv) {
+        const float diff = xv - bv;
+        acc += diff * diff;
+    };
+    if constexpr (VEC4) {
+#pragma unroll 8
+        for (int j = 0; j < d; j += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(row + j);
+            add(x[j], v.x);
+            add(x[j + 1], v.y);
+            add(x[j + 2], v.z);
+            add(x[j + 3], v.w);
+        }
+    } else {
+#pragma unroll 8
+        for (int j = 0; j < d; ++j) add(x[j], row[j]);
+    }
+    return acc;
+}
+
+enum class Read { kFloats, kRows, kSlices };  // a lane's row by 4- or by 16-byte loads, or slices
+
+template <int S, Read READ>
 __global__ void __launch_bounds__(kMaxRerankWaves * WAVE) rerank_kernel(RerankArgs a) {
 #pragma clang fp contract(off)
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -86,39 +110,43 @@ __global__ void __launch_bounds__(kMaxRerankWaves * WAVE) rerank_kernel(RerankAr
         bad |= id >= a.n;  // an id past the base: reported, never read
         const bool use = id >= 0 && id < a.n;
         float acc = 0.f;
-        SliceLoader<VEC4> next;
-        next.load(a.base, a.d, id, use, 0, lane);
-        for (int first = 0; first < a.d; first += kSliceFloats) {
-            wave_lds_fence();  // the previous slice has been read
-            next.store(slice, lane);
-            wave_lds_fence();
-            if (first + kSliceFloats < a.d) next.load(a.base, a.d, id, use, first + kSliceFloats, lane);
-            auto chunk = [&](int c) {
-                return *reinterpret_cast<const float4*>(slice + (lane * 8 + (c ^ ((lane >> 1) & 7))) * 4);
-            };
-            auto add = [&](float xv, float bv) {
-                const float diff = xv - bv;
-                acc += diff * diff;
-            };
-            const int width = a.d - first;
-            if (width >= kSliceFloats) {
+        if constexpr (READ != Read::kSlices) {
+            if (use) acc = row_distance<READ == Read::kRows>(x, a.base + static_cast<int64_t>(id) * a.d, a.d);
+        } else {
+            SliceLoader next;
+            next.load(a.base, a.d, id, use, 0, lane);
+            for (int first = 0; first < a.d; first += kSliceFloats) {
+                wave_lds_fence();  // the previous slice has been read
+                next.store(slice, lane);
+                wave_lds_fence();
+                if (first + kSliceFloats < a.d) next.load(a.base, a.d, id, use, first + kSliceFloats, lane);
+                auto chunk = [&](int c) {
+                    return *reinterpret_cast<const float4*>(slice + (lane * 8 + (c ^ ((lane >> 1) & 7))) * 4);
+                };
+                auto add = [&](float xv, float bv) {
+                    const float diff = xv - bv;
+                    acc += diff * diff;
+                };
+                const int width = a.d - first;
+                if (width >= kSliceFloats) {
 #pragma unroll
-                for (int c = 0; c < kSliceFloats / 4; ++c) {
-                    const float4 v = chunk(c);
-                    const float* xs = x + first + c * 4;
-                    add(xs[0], v.x);
-                    add(xs[1], v.y);
-                    add(xs[2], v.z);
-                    add(xs[3], v.w);
-                }
-            } else {
-                for (int c = 0; c * 4 < width; ++c) {
-                    const float4 v = chunk(c);
-                    const float* xs = x + first + c * 4;
-                    add(xs[0], v.x);
-                    if (c * 4 + 1 < width) add(xs[1], v.y);
-                    if (c * 4 + 2 < width) add(xs[2], v.z);
-                    if (c * 4 + 3 < width) add(xs[3], v.w);
+                    for (int c = 0; c < kSliceFloats / 4; ++c) {
+                        const float4 v = chunk(c);
+                        const float* xs = x + first + c * 4;
+                        add(xs[0], v.x);
+                        add(xs[1], v.y);
+                        add(xs[2], v.z);
+                        add(xs[3], v.w);
+                    }
+                } else {
+                    for (int c = 0; c * 4 < width; ++c) {
+                        const float4 v = chunk(c);
+                        const float* xs = x + first + c * 4;
+                        add(xs[0], v.x);
+                        add(xs[1], v.y);
+                        add(xs[2], v.z);
+                        add(xs[3], v.w);
+                    }
                 }
             }
         }
@@ -151,9 +179,15 @@ hipError_t launch_rerank(const RerankArgs& a, hipStream_t stream) {
     constexpr int64_t kMaxBlocks = int64_t{1} << 22;
     const int waves = static_cast<int>(a.r < WAVE * kMaxRerankWaves ? (a.r + WAVE - 1) / WAVE : kMaxRerankWaves);
     const dim3 threads(static_cast<unsigned>(waves * WAVE));
-    const size_t lds = static_cast<size_t>(waves) * kSliceBytes;  // also holds the wave lists (K <= 128 pairs a wave)
-    static_assert(2 * WAVE * sizeof(Pair) <= kSliceBytes, "a wave's list fits its slice buffer");
+    // Slices where rows are whole halves of lines and a wave takes more than one round of 64 candidates (short rows: more
+    // than one wave's), or where long rows come in numbers that fill the memory's bandwidth.
     const bool vec4 = a.d % 4 == 0 && reinterpret_cast<uintptr_t>(a.base) % 16 == 0;
+    const bool slices = vec4 && a.d % 16 == 0 &&
+                        (a.r > (a.d <= 32 ? WAVE : WAVE * kMaxRerankWaves) ||
+                         (a.d >= 384 && a.r > WAVE && a.nq >= (int64_t{1} << 24) / (a.r * a.d)));
+    // The slices' buffers also hold the wave lists (K <= 128 pairs a wave); without slices the lists alone.
+    const size_t lds = static_cast<size_t>(waves) * (slices ? kSliceBytes : a.K * sizeof(Pair));
+    static_assert(2 * WAVE * sizeof(Pair) <= kSliceBytes, "a wave's list fits its slice buffer");
     for (int64_t q0 = 0; q0 < a.nq; q0 += kMaxBlocks) {
         RerankArgs b = a;
         b.nq = a.nq - q0 < kMaxBlocks ? a.nq - q0 : kMaxBlocks;
@@ -161,13 +195,14 @@ hipError_t launch_rerank(const RerankArgs& a, hipStream_t stream) {
         if (a.candidates) b.candidates = a.candidates + q0 * a.r;
         b.out = a.out + q0 * a.k;
         const dim3 grid(static_cast<unsigned>(b.nq));
-        if (a.K <= WAVE) {
-            if (vec4) hipLaunchKernelGGL((rerank_kernel<1, true>), grid, threads, lds, stream, b);
-            else hipLaunchKernelGGL((rerank_kernel<1, false>), grid, threads, lds, stream, b);
-        } else {
-            if (vec4) hipLaunchKernelGGL((rerank_kernel<2, true>), grid, threads, lds, stream, b);
-            else hipLaunchKernelGGL((rerank_kernel<2, false>), grid, threads, lds, stream, b);
-        }
+        auto launch = [&](auto sc) {
+            constexpr int S = decltype(sc)::value;
+            if (slices) hipLaunchKernelGGL((rerank_kernel<S, Read::kSlices>), grid, threads, lds, stream, b);
+            else if (vec4) hipLaunchKernelGGL((rerank_kernel<S, Read::kRows>), grid, threads, lds, stream, b);
+            else hipLaunchKernelGGL((rerank_kernel<S, Read::kFloats>), grid, threads, lds, stream, b);
+        };
+        if (a.K <= WAVE) launch(std::integral_constant<int, 1>{});
+        else launch(std::integral_constant<int, 2>{});
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
