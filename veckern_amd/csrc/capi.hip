@@ -280,7 +280,7 @@ struct vk_searcher {
     DeviceBuffer<uint8_t> codes, codes_il;
     DeviceBuffer<uint4> heads;             // the first codes of the sorted layout, for scans that abandon tiles
     bool have_heads = false;
-    bool codes_alike = false;              // the codes repeat within tiles (choose_abandon)
+    bool codes_alike = false;              // the codes repeat within tiles (ensure_slot_ids)
     int abandon_mode = VK_ABANDON_AUTO;
     vk_scan_kernel last_kernel{};          // threads = 0 before the first v8/v9 scan
     DeviceBuffer<uint4> codes_v, codes_s;  // words in vector order (v6, v7) and in sorted slot order (v8, v9)
@@ -328,34 +328,23 @@ struct vk_searcher {
             codes_s.ensure(static_cast<size_t>(n_pad) * (m / 16));
             VK_HIP(vk::launch_build_sorted_words(codes.get(), n, static_cast<int>(m), n_pad, slot_ids.get(),
                                                  table_rows.get(), codes_s.get(), stream));
-            choose_abandon();
             have_s = built = true;
         }
         if (vk::plan::uses_sorted_layout(v) && !have_heads && m <= 64 &&
             (abandon_mode == VK_ABANDON_ALWAYS || (abandon_mode == VK_ABANDON_AUTO && codes_alike))) {
             const int words = vk::abandon_head_words(static_cast<int>(m));
-            heads.ensure(static_cast<size_t>(n_pad / 256) * words * vk::WAVE);
-            VK_HIP(vk::launch_build_heads(codes_s.get(), static_cast<int>(m), n_pad, words, heads.get(), stream));
-            have_heads = built = true;
+            try {
+                heads.ensure(static_cast<size_t>(n_pad / 256) * words * vk::WAVE);
+                VK_HIP(vk::launch_build_heads(codes_s.get(), static_cast<int>(m), n_pad, words, heads.get(), stream));
+                have_heads = built = true;
+            } catch (const Failure& f) {
+                // Without room for the head codes the plain scans still run.
+                if (f.code != VK_ERR_OUT_OF_MEMORY || abandon_mode == VK_ABANDON_ALWAYS) throw;
+                (void)hipGetLastError();
+                codes_alike = false;
+            }
         }
         if (built) VK_HIP(hipStreamSynchronize(stream));  // a layout kernel's failure surfaces here, not mid-search
-    }
-
-    // Whether the v8/v9 scans abandon tiles: a tile is dropped when all of its 64 vectors are beyond every bound, which
-    // happens early where the vectors of a tile are close to each other and hardly ever where they are not. Measured as
-    // how far apart the vectors of neighbouring slots are, against vectors half the database apart, in sampled tiles.
-    void choose_abandon() {
-        const int64_t tiles = static_cast<int64_t>(n) / vk::WAVE;
-        if (m > 64 || tiles < 2) return;
-        DeviceBuffer<double> spread;
-        spread.ensure(2);
-        VK_HIP(vk::launch_zero_words(reinterpret_cast<unsigned*>(spread.get()), 4, stream));
-        VK_HIP(vk::launch_tile_spread(codes.get(), slot_ids.get(), centroids.get(), static_cast<int>(m),
-                                      static_cast<int>(d / m), tiles, (tiles + 1023) / 1024, spread.get(), stream));
-        double sums[2] = {0.0, 0.0};
-        VK_HIP(hipMemcpyAsync(sums, spread.get(), sizeof sums, hipMemcpyDeviceToHost, stream));
-        VK_HIP(hipStreamSynchronize(stream));
-        codes_alike = vk::plan::abandon_pays(sums[0], sums[1]);
     }
 
     // The slot order and table rows of the fused scans' layout (slot_order.hpp), for table reads of `lanes` lanes
@@ -393,7 +382,21 @@ struct vk_searcher {
             VK_HIP(hipMemcpyAsync(table_rows.get(), rows.data(), rows.size(), hipMemcpyHostToDevice, stream));
             VK_HIP(vk::launch_slot_place(codes.get(), static_cast<int64_t>(n), static_cast<int>(m), n_pad, lanes,
                                          scratch.get(), bytes, table_rows.get(), slot_ids.get(), stream));
+            // Whether the scans may abandon tiles: a tile is dropped when all of its 64 vectors are beyond every bound,
+            // which happens early where the vectors of a tile are close to each other and hardly ever where they are not.
+            // Measured as how far apart the vectors of neighbouring slots are, against vectors half the database apart, in
+            // sampled tiles; in the sort's scratch, and waited for with the placing.
+            double spread[2] = {0.0, 0.0};
+            const int64_t tiles = static_cast<int64_t>(n) / vk::WAVE;
+            if (tiles >= 2) {
+                double* const sums = reinterpret_cast<double*>(scratch.get());
+                VK_HIP(vk::launch_zero_words(reinterpret_cast<unsigned*>(sums), 4, stream));
+                VK_HIP(vk::launch_tile_spread(codes.get(), slot_ids.get(), centroids.get(), static_cast<int>(m),
+                                              static_cast<int>(d / m), tiles, (tiles + 255) / 256, sums, stream));
+                VK_HIP(hipMemcpyAsync(spread, sums, sizeof spread, hipMemcpyDeviceToHost, stream));
+            }
             VK_HIP(hipStreamSynchronize(stream));
+            codes_alike = vk::plan::abandon_pays(spread[0], spread[1]);
         }
         order_lanes = lanes;
         have_slot_ids = true;

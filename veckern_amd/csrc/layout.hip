@@ -113,8 +113,8 @@ __global__ void build_heads_kernel(const uint32_t* words, int m, int64_t granule
     out[e] = make_uint4(part(0), part(1), part(2), part(3));
 }
 
-// One block per sampled tile of the slot order: squared distances between the codewords of neighbouring lanes' vectors,
-// and of each lane's vector and one half the database away, over the sub-spaces past the sort key.
+// One block per sampled tile of the slot order and four sub-spaces past the sort key (grid y): squared distances between the
+// codewords of neighbouring lanes' vectors, and of each lane's vector and one half the database away.
 __global__ void __launch_bounds__(WAVE)
     tile_spread_kernel(const uint8_t* codes, const uint32_t* slot_ids, const float* centroids, int m, int dsub,
                        int64_t tiles, int64_t stride, double* sums) {
@@ -127,7 +127,8 @@ __global__ void __launch_bounds__(WAVE)
     const uint8_t* const next = row(tile, lane ^ 1);
     const uint8_t* const other = row(far_tile, lane);
     float close = 0.f, apart = 0.f;
-    for (int s = 4; s < m; ++s) {
+    const int s0 = 4 + 4 * static_cast<int>(blockIdx.y);
+    for (int s = s0; s < m && s < s0 + 4; ++s) {
         const float* c = centroids + static_cast<int64_t>(s) * KSUB * dsub;
         for (int j = 0; j < dsub; ++j) {
             const float x = c[own[s] * dsub + j], dn = x - c[next[s] * dsub + j], df = x - c[other[s] * dsub + j];
@@ -160,8 +161,8 @@ hipError_t launch_tile_spread(const uint8_t* codes, const uint32_t* slot_ids, co
                               int64_t tiles, int64_t stride, double* sums, hipStream_t stream) {
     const int64_t blocks = (tiles + stride - 1) / stride;
     if (blocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(tile_spread_kernel, dim3(static_cast<unsigned>(blocks)), dim3(WAVE), 0, stream, codes, slot_ids,
-                       centroids, m, dsub, tiles, stride, sums);
+    hipLaunchKernelGGL(tile_spread_kernel, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>((m - 1) / 4)),
+                       dim3(WAVE), 0, stream, codes, slot_ids, centroids, m, dsub, tiles, stride, sums);
     return hipGetLastError();
 }
 
