@@ -153,9 +153,10 @@ enum vk_abandon { VK_ABANDON_AUTO = 0, VK_ABANDON_ALWAYS = 1, VK_ABANDON_NEVER =
 int vk_searcher_set_abandon(vk_searcher* s, int mode);
 /* The kernel instance of the last v8/v9 scan: queries per table, tables per block, 64-vector tiles per wave step,
  * compile-time sub-spaces (0: any m), list registers per lane, threads per block, fp16 tables, bulk admission, tile
- * abandonment. VK_ERR_LOGIC before the first such search. No counterpart in the reference; for tests and tools. */
+ * abandonment, blocks that first vote whether abandoning pays (when all find that it does not, the batch is scanned again
+ * without, and that is the last kernel). VK_ERR_LOGIC before the first such search. No counterpart in the reference; for tests and tools. */
 typedef struct vk_scan_kernel {
-    int queries_per_table, tables, tiles_per_step, sub_spaces, list_registers, threads, f16, bulk, abandons;
+    int queries_per_table, tables, tiles_per_step, sub_spaces, list_registers, threads, f16, bulk, abandons, votes;
 } vk_scan_kernel;
 int vk_searcher_last_kernel(const vk_searcher* s, vk_scan_kernel* out);
 

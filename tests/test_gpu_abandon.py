@@ -98,6 +98,44 @@ def test_forced_abandonment_matches_oracle(family, d, m):
                             f"{vk.variant_name(variant)} Q={q} threads={threads} blocks={blocks} k={k} nq={count}")
 
 
+@pytest.mark.parametrize("variant,q,nq", [(V8, 1, 170), (V8, 2, 340), (V8, 4, 1_000), (V9, 8, 1_360)])
+def test_queries_far_from_the_data_go_to_the_plain_scan(variant, q, nq):
+    # A million vectors per block, where the blocks first vote: all leave when the queries are far from every vector, none
+    # does when they are near. The second scan may not cost what abandoning in vain did (Q = 2: 1.59 times the plain scan,
+    # fp16 1.44; measured with the vote 1.14 and 1.07).
+    cent, codes, near = datagen.pq_fixture(20_011, 64, 16, nq, seed=940)
+    codes = np.tile(codes, (50, 1))
+    far = np.random.default_rng(941).standard_normal((nq, 64), dtype=np.float32) * 3
+    d_far = vk.DeviceArray.from_host(far)
+    d_out = vk.DeviceArray(nq * 10 * vk.NEIGHBOR_DTYPE.itemsize)
+
+    def scan_ms():
+        return min(s.search_device(d_far.address, nq, 10, variant, d_out.address).scan_ms for _ in range(8))
+
+    try:
+        with vk.PQSearcher(cent, codes, 64) as s:
+            s.set_tuning(vk.Tuning(queries_per_block=q))
+            results, times = {}, {}
+            for mode in (vk.Abandon.Never, vk.Abandon.Auto):
+                s.set_abandon(mode)
+                for name, x in (("far", far), ("near", near), ("mixed", np.concatenate([near[:nq // 2], far[nq // 2:]])),
+                                ("far", far)):
+                    dist, ids, _ = s.search(x, 10, variant)
+                    kernel = s.last_kernel()
+                    assert kernel.abandons == kernel.votes == (mode == vk.Abandon.Auto and name != "far"), (name, kernel)
+                    if mode == vk.Abandon.Never:
+                        results[name] = dist, ids
+                    else:
+                        assert (ids == results[name][1]).all() and (dist == results[name][0]).all(), name
+                times[mode] = scan_ms()
+            got = d_out.download(np.empty((nq, 10), dtype=vk.NEIGHBOR_DTYPE))
+            assert (got["id"] == results["far"][1]).all()
+            assert times[vk.Abandon.Auto] < 1.32 * times[vk.Abandon.Never], times
+    finally:
+        d_far.free()
+        d_out.free()
+
+
 def test_abandonment_modes():
     cent, codes, queries = datagen.pq_fixture(140_003, 64, 16, 4, seed=930)
     exp = orc.adc_search(cent, 64, codes, queries, 10)

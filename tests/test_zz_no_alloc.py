@@ -95,6 +95,18 @@ def test_noalloc_abandoned_tiles(variant, q):
             assert_same(expected, new, f"oracle nq={nq} blocks={blocks}")
 
 
+def test_noalloc_queries_far_from_the_data():
+    # The blocks of the abandoning scan vote to leave, and the batch is scanned again without abandonment.
+    centroids, codes, near = datagen.pq_fixture(20_011, 64, 16, 340, seed=29)
+    far = np.random.default_rng(30).standard_normal((340, 64), dtype=np.float32) * 3
+    with vk.PQSearcher(centroids, np.tile(codes, (50, 1)), 64) as s:
+        s.set_tuning(vk.Tuning(queries_per_block=2))
+        for queries, leaves in ((near, False), (far, True), (far, True), (near, False)):
+            ref, new, _, _ = search_pair(s, queries, 10, vk.ScanVariant.FusedWarp)
+            assert s.last_kernel().abandons != leaves
+            assert_same(ref, new, f"leaves={leaves}")
+
+
 @pytest.mark.parametrize("nq,k", [(1025, 64), (1040, 64), (1500, 64), (2048, 64), (2048, 10)])
 def test_noalloc_takes_batches_of_alike_codes_that_fit_the_plain_scan(nq, k):
     # Codes that repeat within tiles, more slabs than CUs: blocks of 1024 threads cross slab boundaries, and their

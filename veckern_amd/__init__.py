@@ -81,7 +81,8 @@ class _LaunchShape(ctypes.Structure):
 class _ScanKernel(ctypes.Structure):
     _fields_ = [("queries_per_table", ctypes.c_int), ("tables", ctypes.c_int), ("tiles_per_step", ctypes.c_int),
                 ("sub_spaces", ctypes.c_int), ("list_registers", ctypes.c_int), ("threads", ctypes.c_int),
-                ("f16", ctypes.c_int), ("bulk", ctypes.c_int), ("abandons", ctypes.c_int)]
+                ("f16", ctypes.c_int), ("bulk", ctypes.c_int), ("abandons", ctypes.c_int),
+                ("votes", ctypes.c_int)]
 
 
 class _DeviceInfo(ctypes.Structure):
@@ -235,13 +236,14 @@ class ScanKernel:
     f16: bool
     bulk: bool
     abandons: bool
+    votes: bool
 
     @property
     def symbol(self) -> str:
         """The kernel's name as a profiler prints it."""
         numbers = (self.queries_per_table, self.tables, self.tiles_per_step, self.sub_spaces, self.list_registers,
                    self.threads)
-        flags = (self.f16, False, self.bulk, self.abandons)
+        flags = (self.f16, False, self.bulk, self.abandons, self.votes)
         return f"fused_wave_kernel_t<{', '.join([str(n) for n in numbers] + [str(f).lower() for f in flags])}>"
 
 
@@ -375,7 +377,7 @@ class PQSearcher:
         k = _ScanKernel()
         _check(library().vk_searcher_last_kernel(self._h, ctypes.byref(k)))
         return ScanKernel(k.queries_per_table, k.tables, k.tiles_per_step, k.sub_spaces, k.list_registers, k.threads,
-                          bool(k.f16), bool(k.bulk), bool(k.abandons))
+                          bool(k.f16), bool(k.bulk), bool(k.abandons), bool(k.votes))
 
     def search(self, queries: np.ndarray, k: int, variant: int = ScanVariant.FusedWarp):
         """Returns (dist [nq, k] float32, ids [nq, k] int32, Timings)."""

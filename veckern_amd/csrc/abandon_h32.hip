@@ -2,7 +2,7 @@
 #include "fused_wave.inl"
 
 namespace vk {
-WaveScanKernel abandon_kernel_h32(int q, int threads) {
-    return select_abandon_kernel<32, true>(q, threads);
+WaveScanKernel abandon_kernel_h32(int q, int threads, bool vote) {
+    return select_abandon_kernel<32, true>(q, threads, vote);
 }
 }  // namespace vk

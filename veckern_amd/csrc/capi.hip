@@ -35,21 +35,21 @@ WaveScanKernel fused_wave_kernel_h48(int qg, int ng, int ilp, int segments, bool
 WaveScanKernel fused_wave_kernel_h64(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 WaveScanKernel fused_wave_kernel_hx(int qg, int ng, int ilp, int segments, bool bulk, int threads);
 
-WaveScanKernel abandon_kernel_m16(int q, int threads);
-WaveScanKernel abandon_kernel_m32(int q, int threads);
-WaveScanKernel abandon_kernel_m48(int q, int threads);
-WaveScanKernel abandon_kernel_m64(int q, int threads);
-WaveScanKernel abandon_kernel_h16(int q, int threads);
-WaveScanKernel abandon_kernel_h32(int q, int threads);
-WaveScanKernel abandon_kernel_h48(int q, int threads);
-WaveScanKernel abandon_kernel_h64(int q, int threads);
+WaveScanKernel abandon_kernel_m16(int q, int threads, bool vote);
+WaveScanKernel abandon_kernel_m32(int q, int threads, bool vote);
+WaveScanKernel abandon_kernel_m48(int q, int threads, bool vote);
+WaveScanKernel abandon_kernel_m64(int q, int threads, bool vote);
+WaveScanKernel abandon_kernel_h16(int q, int threads, bool vote);
+WaveScanKernel abandon_kernel_h32(int q, int threads, bool vote);
+WaveScanKernel abandon_kernel_h48(int q, int threads, bool vote);
+WaveScanKernel abandon_kernel_h64(int q, int threads, bool vote);
 
-WaveScanKernel abandon_kernel(int q, int m, bool f16, int threads) {
+WaveScanKernel abandon_kernel(int q, int m, bool f16, int threads, bool vote) {
     switch (m) {
-        case 16: return f16 ? abandon_kernel_h16(q, threads) : abandon_kernel_m16(q, threads);
-        case 32: return f16 ? abandon_kernel_h32(q, threads) : abandon_kernel_m32(q, threads);
-        case 48: return f16 ? abandon_kernel_h48(q, threads) : abandon_kernel_m48(q, threads);
-        case 64: return f16 ? abandon_kernel_h64(q, threads) : abandon_kernel_m64(q, threads);
+        case 16: return f16 ? abandon_kernel_h16(q, threads, vote) : abandon_kernel_m16(q, threads, vote);
+        case 32: return f16 ? abandon_kernel_h32(q, threads, vote) : abandon_kernel_m32(q, threads, vote);
+        case 48: return f16 ? abandon_kernel_h48(q, threads, vote) : abandon_kernel_m48(q, threads, vote);
+        case 64: return f16 ? abandon_kernel_h64(q, threads, vote) : abandon_kernel_m64(q, threads, vote);
         default: return WaveScanKernel{};
     }
 }
@@ -282,6 +282,9 @@ struct vk_searcher {
     bool have_heads = false;
     bool codes_alike = false;              // the codes repeat within tiles (ensure_slot_ids)
     int abandon_mode = VK_ABANDON_AUTO;
+    PinnedBuffer<unsigned> left;           // written by an abandoning scan whose blocks all left (WavePlan::vote)
+    DeviceBuffer<unsigned> votes;          // two words, used in turn
+    unsigned vote_turn = 0;
     vk_scan_kernel last_kernel{};          // threads = 0 before the first v8/v9 scan
     DeviceBuffer<uint4> codes_v, codes_s;  // words in vector order (v6, v7) and in sorted slot order (v8, v9)
     DeviceBuffer<uint32_t> slot_ids;        // the sorted slot order: the vector id of each slot (m % 16 == 0 only)
@@ -334,6 +337,10 @@ struct vk_searcher {
             (abandon_mode == VK_ABANDON_ALWAYS || (abandon_mode == VK_ABANDON_AUTO && codes_alike))) {
             const int words = vk::abandon_head_words(static_cast<int>(m));
             try {
+                left.ensure(1);
+                *left.get() = 0;
+                votes.ensure(2);
+                VK_HIP(vk::launch_zero_words(votes.get(), 2, stream));
                 heads.ensure(static_cast<size_t>(n_pad / 256) * words * vk::WAVE);
                 VK_HIP(vk::launch_build_heads(codes_s.get(), static_cast<int>(m), n_pad, words, heads.get(), stream));
                 have_heads = built = true;
@@ -434,6 +441,7 @@ struct vk_searcher {
         size_t smem = 0;
         int q = 1, ilp = 1, K = 0, per_cu = 1, lists_per_block = 1;
         vk::plan::Partition part;
+        bool vote = false;      // the blocks may all leave: the batch is then searched by a plan without abandonment
         vk_scan_kernel id{};    // the instance
         size_t part_pairs = 0;  // partial-list pairs: [slabs][q][max_slots][lists_per_block][K]
     };
@@ -515,8 +523,20 @@ struct vk_searcher {
                 bulk_lists = true;
             }
         }
+        // A vote needs every block's, so all of them resident.
+        if (abandon && !always && w.part.grid <= static_cast<int64_t>(w.per_cu) * info.sm_count &&
+            vk::plan::block_vectors(w.part, w.ilp) >= vk::plan::vote_vectors(w.q)) {
+            const vk::WaveScanKernel voting = vk::abandon_kernel(w.q, static_cast<int>(m), f16, w.kern.threads, true);
+            int voting_per_cu = 0;
+            if (voting.fn)
+                VK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&voting_per_cu, voting.fn, voting.threads, w.smem));
+            if (voting_per_cu == w.per_cu) {
+                w.kern = voting;
+                w.vote = true;
+            }
+        }
         w.id = vk_scan_kernel{qg, ng, w.ilp, w.kern.dynamic_lds ? 0 : static_cast<int>(m), segments, w.kern.threads,
-                              f16, bulk_lists, abandon};
+                              f16, bulk_lists, abandon, w.vote};
         // Up to 8 blocks per slab every wave leaves its own partial lists; beyond that the block merges its wave
         // lists first, which keeps the final merge of a slab to at most max(64, blocks per slab) lists per query.
         w.lists_per_block = w.part.max_slots > 8 ? 1 : w.kern.threads / vk::WAVE;
@@ -560,15 +580,41 @@ struct vk_searcher {
         a.part = part_buf;
         a.counters = counter_buf;
         a.bounds = bound_buf;
+        if (w.vote) {
+            a.vote = votes.get() + vote_turn % 2;
+            a.next_vote = votes.get() + (vote_turn + 1) % 2;
+            ++vote_turn;
+            a.left = left.get();
+        }
         a.heads = heads.get();
         a.out = d_out;
         VK_HIP(w.kern.launch(a, static_cast<int>(w.part.grid), w.smem, stream));
     }
 
+    // After a scan with a vote has completed: whether its blocks left (asked once).
+    bool blocks_left(const WavePlan& w) {
+        if (!w.vote || *left.get() == 0) return false;
+        *left.get() = 0;
+        return true;
+    }
+
+    // Before a scan, when a call may have raised between a launch and the stream's completion: waits for it and clears what
+    // it left of a vote.
+    void clear_votes() {
+        if (votes.empty()) return;
+        VK_HIP(hipStreamSynchronize(stream));
+        *left.get() = 0;
+        VK_HIP(vk::launch_zero_words(votes.get(), 2, stream));
+    }
+
     // d_q: device queries of this batch; writes b x kk results to d_out, with the searcher's own scratch buffers.
     // The LUT and the final merge are inside scan_ms.
-    void run_wave(const float* d_q, size_t b, size_t kk, bool f16, Pair* d_out, vk_timings* t, StageClock& clock) {
-        const WavePlan w = plan_wave(b, kk, f16);
+    // Returns whether the blocks may leave; the caller then asks blocks_left when the stream has completed and runs the batch
+    // again without abandonment if so.
+    WavePlan run_wave(const float* d_q, size_t b, size_t kk, bool f16, Pair* d_out, vk_timings* t, StageClock& clock,
+                      bool may_abandon = true) {
+        const WavePlan w = plan_wave(b, kk, f16, may_abandon);
+        if (counters_dirty) clear_votes();
         part.ensure(w.part_pairs);
         const size_t slabs = static_cast<size_t>(w.part.slabs);
         ensure_counters(slabs + slabs * static_cast<size_t>(w.q));
@@ -576,6 +622,15 @@ struct vk_searcher {
         clock.time(&t->scan_ms, [&] {
             launch_wave(w, d_q, b, kk, d_out, part.get(), counters.get(), counters.get() + slabs);
         });
+        return w;
+    }
+
+    // When a batch's stream has completed: runs it again without abandonment if its blocks left. False: nothing to do.
+    bool run_again(const WavePlan& w, const float* d_q, size_t b, size_t kk, Pair* d_out, vk_timings* t, StageClock& clock) {
+        if (!blocks_left(w)) return false;
+        counters_dirty = false;  // the scan completed; no counter was touched
+        run_wave(d_q, b, kk, w.id.f16 != 0, d_out, t, clock, false);
+        return true;
     }
 
     // Per-slab completion counters and per-query shared bounds of the wave-list scan (`slabs`: words of both). The
@@ -673,11 +728,13 @@ struct vk_searcher {
         clock.time(&t->select_ms, [&] { VK_HIP(vk::launch_select(s, static_cast<int>(b), stream)); });
     }
 
-    void run_variant(int v, const float* d_q, size_t b, size_t kk, Pair* d_out, vk_timings* t, StageClock& clock) {
+    // Returns the plan of a v8/v9 batch (run_again), an empty one otherwise.
+    WavePlan run_variant(int v, const float* d_q, size_t b, size_t kk, Pair* d_out, vk_timings* t, StageClock& clock) {
         if (v == VK_V8_FUSED_WARP || v == VK_V9_FUSED_WARP_F16)
             return run_wave(d_q, b, kk, v == VK_V9_FUSED_WARP_F16, d_out, t, clock);
-        if (vk_is_fused(v)) return run_thread(v, d_q, b, kk, d_out, t, clock);
-        run_unfused(v, d_q, b, kk, d_out, t, clock);
+        if (vk_is_fused(v)) run_thread(v, d_q, b, kk, d_out, t, clock);
+        else run_unfused(v, d_q, b, kk, d_out, t, clock);
+        return {};
     }
 
     void check_search(size_t kk, int v) const {
@@ -740,12 +797,16 @@ struct vk_searcher {
                 VK_HIP(hipMemcpyAsync(queries.get(), staged_q.get(), b * d * sizeof(float), hipMemcpyHostToDevice,
                                       stream));
             });
-            run_variant(v, queries.get(), b, kk, out.get(), t, clock);
-            clock.time(&t->transfer_ms, [&] {
-                VK_HIP(hipMemcpyAsync(staged_out.get(), out.get(), b * kk * sizeof(Pair), hipMemcpyDeviceToHost,
-                                      stream));
-            });
-            clock.settle();
+            const WavePlan w = run_variant(v, queries.get(), b, kk, out.get(), t, clock);
+            auto copy_out = [&] {
+                clock.time(&t->transfer_ms, [&] {
+                    VK_HIP(hipMemcpyAsync(staged_out.get(), out.get(), b * kk * sizeof(Pair), hipMemcpyDeviceToHost,
+                                          stream));
+                });
+                clock.settle();
+            };
+            copy_out();
+            if (run_again(w, queries.get(), b, kk, out.get(), t, clock)) copy_out();
             counters_dirty = false;
             std::memcpy(host_out + q0 * kk, staged_out.get(), b * kk * sizeof(Pair));
         }
@@ -759,8 +820,10 @@ struct vk_searcher {
         const size_t batch = query_batch(v);
         for (size_t q0 = 0; q0 < nq; q0 += batch) {
             const size_t b = std::min(batch, nq - q0);
-            run_variant(v, d_q + q0 * d, b, kk, reinterpret_cast<Pair*>(d_out + q0 * kk), t, clock);
+            Pair* const to = reinterpret_cast<Pair*>(d_out + q0 * kk);
+            const WavePlan w = run_variant(v, d_q + q0 * d, b, kk, to, t, clock);
             clock.settle();
+            if (run_again(w, d_q + q0 * d, b, kk, to, t, clock)) clock.settle();
             counters_dirty = false;
         }
     }
@@ -814,16 +877,31 @@ struct vk_searcher {
         if (!dev.counters_clean)
             VK_HIP(vk::launch_zero_words(counter_buf, static_cast<int64_t>(kNoAllocCounterBytes / sizeof(unsigned)),
                                          stream));
+        if (!dev.counters_clean) clear_votes();
         dev.counters_clean = false;  // until the stream has completed every launch below
         for (size_t q0 = 0; q0 < nq; q0 += batch) {
             const size_t b = std::min(batch, nq - q0);
-            const WavePlan w = plan(b);
+            WavePlan w = plan(b);
+            WavePlan plain;
+            if (w.vote) {
+                plain = plan_wave(b, kk, f16, false);
+                if (part_bytes(plain) > kNoAllocScratchBytes - kNoAllocCounterBytes) {  // no room to leave to: no vote
+                    w.kern = vk::abandon_kernel(w.q, static_cast<int>(m), f16, w.kern.threads);
+                    w.vote = false;
+                    w.id.votes = 0;
+                }
+            }
             // The shared bounds sit behind the counters where both fit; without them the slab's blocks scan with
             // their own bounds only (same results).
             const size_t slabs = static_cast<size_t>(w.part.slabs);
             const bool fit = (slabs + slabs * static_cast<size_t>(w.q)) * sizeof(unsigned) <= kNoAllocCounterBytes;
             launch_wave(w, d_q + q0 * d, b, kk, reinterpret_cast<Pair*>(d_out + q0 * kk), part_buf, counter_buf,
                         fit ? counter_buf + slabs : nullptr);
+            if (!w.vote) continue;
+            VK_HIP(hipStreamSynchronize(stream));
+            if (blocks_left(w))
+                launch_wave(plain, d_q + q0 * d, b, kk, reinterpret_cast<Pair*>(d_out + q0 * kk), part_buf, counter_buf,
+                            nullptr);
         }
         VK_HIP(hipStreamSynchronize(stream));
         dev.counters_clean = true;

@@ -576,6 +576,33 @@ __device__ __forceinline__ int64_t slab_of(const int64_t* slab_gran, int64_t sla
     return lo;
 }
 
+// One vote of the grid on leaving an abandoning scan (one thread of each block, once): true in every block if every block
+// asked to leave, false in every block otherwise. The word counts the blocks that asked to leave; kStay is set by a block that
+// did not, or that has waited too long for the rest (a bounded wait: blocks may not all be resident), and never after the
+// count is complete.
+__device__ __forceinline__ bool vote_to_leave(const WaveScanArgs& a, bool leave) {
+    constexpr unsigned kStay = 1u << 31;
+    constexpr int kPolls = 64;  // about a microsecond each
+    const unsigned all = gridDim.x;
+    if (!leave) {
+        __hip_atomic_fetch_or(a.vote, kStay, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+    }
+    unsigned word = __hip_atomic_fetch_add(a.vote, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+    for (int poll = 0; poll < kPolls && word < all; ++poll) {
+        __builtin_amdgcn_s_sleep(4);
+        word = __hip_atomic_load(a.vote, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    while (word < all) {  // waited too long: stay, unless the count has become complete (it only grows: this ends)
+        if (__hip_atomic_compare_exchange_strong(a.vote, &word, word | kStay, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
+            return false;
+    }
+    if (word != all) return false;  // kStay
+    __hip_atomic_store(a.left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return true;
+}
+
 // IVF (one query per slab, QS = 1): the scan runs over inverted lists. Slab q * a.nprobe + p is the p-th list probed
 // by query q; slabs are in query-major order, so a query's probed lists form one run of consecutive slabs,
 // granules [a.query_gran[q], a.query_gran[q + 1]) of the balanced partition (a.query_gran[nq] = total). Slab s covers
@@ -584,7 +611,8 @@ __device__ __forceinline__ int64_t slab_of(const int64_t* slab_gran, int64_t sla
 // looking it up by list), and the vector ids come from a.ids (-1 on padding). A block
 // gathers a query's tables and starts its lists once per run and writes them once, at the end of the run (or of
 // its range); a separate merge kernel combines the partial lists of each query.
-template <int QG, int NG, int U, int M, int S, int T, bool F16, bool IVF, bool BULK, bool ABANDON = false>
+template <int QG, int NG, int U, int M, int S, int T, bool F16, bool IVF, bool BULK, bool ABANDON = false,
+          bool VOTE = false>
 __global__ void __launch_bounds__(T)
     __attribute__((amdgpu_waves_per_eu(wave_kernel_waves_per_simd<QG, NG, M, T, F16>())))
     fused_wave_kernel_t(WaveScanArgs a) {
@@ -628,6 +656,20 @@ __global__ void __launch_bounds__(T)
     // through, two more sub-spaces (10 VALU per tile) stop nearly all of those.
     constexpr int kCheck = M == 16 && QS >= 4 ? 6 : M / 4;
     __shared__ unsigned block_bound[QS];  // raw bits of a distance >= 0 or +inf: unsigned order is float order
+    // Queries far from every vector, or codes less alike than the layout's sample, leave most tiles alive, and a tile that
+    // stays alive costs more here than in the plain scan (its codes are read twice, one tile at a time): 1M vectors, queries
+    // from no component of the mixture, m = 16: 635 -> 793 us (680 queries, Q = 4), 379 -> 599 (340, Q = 2), 332 -> 560 (170,
+    // Q = 1), fp16 tables 1218 -> 1750 (1360, Q = 8); m = 32 at most 1.18, m = 48 and 64 at most 1.07 of the plain scan's time.
+    // VOTE (m = 16): each block first sums half of the sub-spaces of kSample tiles per wave, spread over its range, and votes;
+    // if every block finds more than kMostLive of them alive, all leave and the host launches the plain scan (691, 430, 377
+    // and 1299 us). All of them, since one block's plain scan takes as long as the whole grid's. An instance of its own, as
+    // the sample's registers cost the scan of few vectors per block up to 12 % (Q = 1). Not both loops in one kernel, nor a
+    // count kept in the loop: the registers they need spill (both loops, fp16 tables, 8 queries of the mixture: 560 -> 1496
+    // us; the count, Q = 4: 315 -> 497).
+    constexpr int kSample = 2;
+    constexpr unsigned kMostLive = W * kSample * 3 / 4;
+    __shared__ unsigned sampled_live;
+    __shared__ bool all_leave;
     __shared__ int share_rank[kPrune ? QS : 1][W];  // raw bits of the ceil(K/W)-th best of each wave's best tile
     // Long lists (K > 64), and the bulk instances (few vectors per block): per (query, wave), the distance of the
     // wave list's entry ceil(K/W) - 1 for the current slab (raw bits of a distance >= 0, so unsigned order is float
@@ -723,6 +765,10 @@ __global__ void __launch_bounds__(T)
     uint4 next_words[kPrefetch ? U : 1];
     SlotIds<U> next_ids;
 
+    if constexpr (VOTE) {
+        if (b == 0 && tid == 0)
+            __hip_atomic_store(a.next_vote, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     for (int64_t item = start; item < end;) {
         // The slab holding `item` and its granules [slab_first, slab_next) in the balanced partition.
         int64_t slab, slab_first, slab_next;
@@ -797,6 +843,7 @@ __global__ void __launch_bounds__(T)
                 for (int t = tid; t < QS * W; t += T) (&rank_bound[0][0])[t] = 0x7f800000u;  // +inf
             if (!IVF && tid == 0) next_gran = kPrune ? 2 * W : W;
             if (kPrune && tid < QS) block_bound[tid] = 0x7f800000u;  // +inf
+            if (VOTE && tid == 0) sampled_live = 0;
             if constexpr (kPrune)
                 for (int t = tid; t < QS * W; t += T) (&share_rank[0][0])[t] = 0x7f800000;
             __syncthreads();
@@ -1224,6 +1271,27 @@ __global__ void __launch_bounds__(T)
                 if (lane == 0) atomicMin(&block_bound[i], static_cast<unsigned>(bound));
             }
         };
+        // The sampled tiles that are alive after half of the sub-spaces, with the bounds found before the scan.
+        auto sample_tiles = [&]() __attribute__((always_inline)) {
+            unsigned live_count = 0;  // wave-uniform
+            const int64_t span_tiles = (g_hi - g_lo) * U;
+#pragma unroll 1
+            for (int i = 0; i < kSample; ++i) {
+                const int64_t tile = g_lo * U + span_tiles * (i * W + wave) / (kSample * W);
+                uint4 cw[WORDS];
+#pragma unroll
+                for (int w = 0; w < (WORDS + 1) / 2; ++w) cw[w] = a.codes[(tile * WORDS + w) * WAVE + lane];
+                float sum[QS];
+                span(std::integral_constant<int, 0>{}, std::integral_constant<int, M / 2>{},
+                     [&](int s) __attribute__((always_inline)) { return word_part(cw[s / 16], s % 16); }, sum);
+                uint64_t any = 0;
+#pragma unroll
+                for (int q = 0; q < QS; ++q)
+                    any |= __builtin_amdgcn_ballot_w64(sum[q] <= __uint_as_float(block_bound[q]) && live[q]);
+                live_count += any != 0;
+            }
+            if (lane == 0) atomicAdd(&sampled_live, live_count);
+        };
         auto prune_step = [&]() __attribute__((always_inline)) {
             constexpr int kHalf = M / 2;
             unsigned grab = 0;
@@ -1364,6 +1432,15 @@ __global__ void __launch_bounds__(T)
         }
         if constexpr (kPrune) {
             first_bounds();
+            if constexpr (VOTE) {
+                if (item == start) {  // block-uniform
+                    sample_tiles();
+                    __syncthreads();
+                    if (tid == 0) all_leave = vote_to_leave(a, sampled_live > kMostLive);
+                    __syncthreads();
+                    if (all_leave) break;
+                }
+            }
             if (g < g_hi) load_heads(g);
             while (g < g_hi) prune_step();
         } else {
@@ -1466,21 +1543,21 @@ __global__ void __launch_bounds__(T)
     }
 }
 
-template <int QG, int NG, int U, int M, int S, int T, bool F16, bool IVF, bool BULK, bool ABANDON>
+template <int QG, int NG, int U, int M, int S, int T, bool F16, bool IVF, bool BULK, bool ABANDON, bool VOTE>
 hipError_t launch_fused_wave_t(const WaveScanArgs& a, int grid, size_t smem, hipStream_t stream) {
-    hipLaunchKernelGGL((fused_wave_kernel_t<QG, NG, U, M, S, T, F16, IVF, BULK, ABANDON>), dim3(grid), dim3(T), smem,
+    hipLaunchKernelGGL((fused_wave_kernel_t<QG, NG, U, M, S, T, F16, IVF, BULK, ABANDON, VOTE>), dim3(grid), dim3(T), smem,
                        stream, a);
     return hipGetLastError();
 }
 
 template <int QG, int NG, int U, int M, int S, bool F16, bool IVF = false, bool BULK = false, int T = 512,
-          bool ABANDON = false>
+          bool ABANDON = false, bool VOTE = false>
 WaveScanKernel make_wave_kernel() {
     WaveScanKernel k;
-    k.fn = reinterpret_cast<const void*>(&fused_wave_kernel_t<QG, NG, U, M, S, T, F16, IVF, BULK, ABANDON>);
+    k.fn = reinterpret_cast<const void*>(&fused_wave_kernel_t<QG, NG, U, M, S, T, F16, IVF, BULK, ABANDON, VOTE>);
     k.threads = T;
     k.dynamic_lds = M == 0;
-    k.launch = &launch_fused_wave_t<QG, NG, U, M, S, T, F16, IVF, BULK, ABANDON>;
+    k.launch = &launch_fused_wave_t<QG, NG, U, M, S, T, F16, IVF, BULK, ABANDON, VOTE>;
     return k;
 }
 
@@ -1551,19 +1628,21 @@ WaveScanKernel select_wave_kernel(int qg, int ng, int ilp, int segments, bool bu
     return WaveScanKernel{};
 }
 
-// Instances that abandon tiles, for one M and entry type: one table group, lists of up to 64, four tiles per wave step, 1024-thread blocks
-// where kWideBlock holds (more waves share a bound), else 512.
-template <int M, bool F16>
-WaveScanKernel select_abandon_kernel(int q, int threads) {
+// Instances that abandon tiles, for one M and entry type: one table group, lists of up to 64, four tiles per wave step,
+// 1024-thread blocks where kWideBlock holds (more waves share a bound), else 512. vote: the instance whose blocks first vote
+// (M = 16 only).
+template <int M, bool F16, bool VOTE>
+WaveScanKernel make_abandon_kernel(int q, int threads) {
     constexpr int kLds = 160 * 1024;
-#define VK_ABANDON(QG_)                                                                                           \
-    if (q == QG_) {                                                                                              \
-        if constexpr (M * KSUB * Entries<QG_, F16>::kBytes <= kLds) {                                             \
-            if constexpr (kWideBlock<QG_, 1, M, 1, F16>) {                                                       \
-                if (threads == 1024) return make_wave_kernel<QG_, 1, 4, M, 1, F16, false, false, 1024, true>();  \
-            }                                                                                                    \
-            if (threads == 512) return make_wave_kernel<QG_, 1, 4, M, 1, F16, false, false, 512, true>();        \
-        }                                                                                                        \
+#define VK_ABANDON(QG_)                                                                                            \
+    if (q == QG_) {                                                                                               \
+        if constexpr (M * KSUB * Entries<QG_, F16>::kBytes <= kLds) {                                              \
+            if constexpr (kWideBlock<QG_, 1, M, 1, F16>) {                                                        \
+                if (threads == 1024)                                                                              \
+                    return make_wave_kernel<QG_, 1, 4, M, 1, F16, false, false, 1024, true, VOTE>();              \
+            }                                                                                                     \
+            if (threads == 512) return make_wave_kernel<QG_, 1, 4, M, 1, F16, false, false, 512, true, VOTE>();    \
+        }                                                                                                         \
     }
     VK_ABANDON(1)
     VK_ABANDON(2)
@@ -1572,6 +1651,13 @@ WaveScanKernel select_abandon_kernel(int q, int threads) {
         VK_ABANDON(8)
     }
 #undef VK_ABANDON
+    return WaveScanKernel{};
+}
+
+template <int M, bool F16>
+WaveScanKernel select_abandon_kernel(int q, int threads, bool vote) {
+    if (!vote) return make_abandon_kernel<M, F16, false>(q, threads);
+    if constexpr (M == 16) return make_abandon_kernel<M, F16, true>(q, threads);
     return WaveScanKernel{};
 }
 

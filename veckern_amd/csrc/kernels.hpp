@@ -73,6 +73,11 @@ struct WaveScanArgs {
     // [slabs][qg * ng], zero between searches, or nullptr: per query the smallest K-th best distance that a block of
     // the slab has found, as complemented raw bits (so that zero means none and the largest word wins).
     unsigned* bounds;
+    // Voting instances: a zero word in which the blocks vote on leaving (vote_to_leave), the word of the next such launch,
+    // which this one clears, and the word in host memory that says they left (no result was written).
+    unsigned* vote;
+    unsigned* next_vote;
+    unsigned* left;
     const uint4* heads;      // head codes (launch_build_heads) for the instances that abandon tiles
     Pair* out;               // [nq][k]; empty slots become {+inf, -1}
     // Inverted lists (IVF instances only, one query per slab, the plan of launch_ivf_plan); `n_gran`, `total` and
@@ -95,7 +100,8 @@ struct WaveScanKernel {
 
 // The instance that abandons tiles (m = 16, 32, 48, 64; q queries in one table group, K <= 64; 1024 or 512 threads); fn ==
 // nullptr when it is not built.
-WaveScanKernel abandon_kernel(int q, int m, bool f16, int threads);
+// vote: the instance whose blocks first vote on leaving (WaveScanArgs::vote; m = 16).
+WaveScanKernel abandon_kernel(int q, int m, bool f16, int threads, bool vote = false);
 // Returns a kernel with fn == nullptr when the combination is not built. f16: binary16 tables (v9). bulk: the
 // instance with bulk admission into one-register lists (fp32, more than one query per block only). threads: block
 // size, 512 or 1024 (built for four tiles per wave step where two 512-thread blocks' tables fit one CU).

@@ -114,6 +114,13 @@ inline bool bulk_scan(const Partition& p, int ilp) {
 // near vectors than a tile holds, and at k = 100 the plain scan was faster (1M, m = 16: 722 against 787 us).
 constexpr int64_t kAbandonVectors = int64_t{1} << 15;
 
+// Vectors per block from which the blocks of an abandoning scan (q queries per table) first vote whether it pays. The sample
+// and the plain scan launched after they leave cost 25 us and more, which over fewer vectors is as much as abandoning in vain
+// does. us plain, abandoning in vain, leaving (1M vectors, m = 16): Q = 4, 333k vectors per block 286, 329, 350, 500k 381,
+// 444, 444, 1M 635, 793, 691; Q = 2, 250k 171, 203, 217, 333k 185, 259, 241; Q = 1, 333k 162, 242, 212; fp16, Q = 8, 333k
+// 536, 690, 636.
+inline int64_t vote_vectors(int q) { return q == 4 ? 1 << 19 : 1 << 18; }
+
 // Whether scans that abandon tiles pay: the mean squared distance between vectors of one tile (past the sort key),
 // against that between vectors far apart in the slot order. Uniform codes have a ratio of 1 and no tile can be dropped;
 // the Gaussian mixture of the benchmark (1000 components, sigma 0.3) about 0.1.
