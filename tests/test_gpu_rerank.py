@@ -56,11 +56,11 @@ def test_rerank_other_dims_and_ties(d, family):
             assert_same(got_d, got_i, orc.rerank_exact(base, queries, cand, k), f"d={d} {family} k={k}")
 
 
-# Rows read by their own lane, or slices of 64 rows: from 513 candidates (65 for d <= 32) where d % 16 == 0, and for long
-# rows from 2^24 gathered values (384 x 65 x 672).
-@pytest.mark.parametrize("d,r,nq", [(16, 64, 9), (16, 65, 9), (32, 200, 9), (48, 65, 9), (48, 512, 5), (48, 513, 5),
-                                    (100, 700, 5), (130, 700, 5), (200, 1025, 5), (384, 65, 671), (384, 65, 672),
-                                    (400, 600, 71), (960, 10, 40), (960, 300, 59)])
+# Rows read by their own lane, or slices of 64 rows: from 257 candidates, or 65 where the call gathers 2^24 values
+# (384 x 65 x 672), for d % 4 == 0 from d = 16.
+@pytest.mark.parametrize("d,r,nq", [(12, 300, 9), (16, 256, 9), (16, 257, 9), (32, 700, 9), (48, 65, 9), (48, 513, 5),
+                                    (100, 256, 5), (100, 700, 5), (130, 700, 5), (200, 1025, 5), (384, 64, 700),
+                                    (384, 65, 671), (384, 65, 672), (400, 600, 71), (960, 10, 40), (960, 300, 59)])
 def test_rerank_ways_to_read_rows(d, r, nq):
     base, queries, cand = case(65 + d + r, 2_000, d, nq, r)
     with vk.Reranker(base) as rr:

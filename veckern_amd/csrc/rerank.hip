@@ -12,12 +12,13 @@
 //  - rows: a lane reads its own row with 16-byte loads, eight in flight;
 //  - slices: 32 floats of 64 rows at a time, 8 consecutive lanes on a 128-byte slice of a row, through LDS to the lane that
 //    sums them, with the next slice's loads in flight meanwhile. A lane that reads its own row touches a line of its own
-//    with every load, 64 lines per instruction, which costs where many rows are read per wave; a slice costs a pass through
-//    LDS each, 30 in a row for d = 960, and twice the lines where rows are not whole lines.
-// us per call, rows / slices: d = 128, 2000 x 100 34.6 / 35.8, 300 x 1000 56.2 / 45.5, one query x 100 19.0 / 21.4; d = 200,
-// 2000 x 100 47.0 / 53.0; d = 130, 2000 x 100 54.6 / 72.1; d = 384, 1000 x 1000 297 / 244; d = 960, 2000 x 10 37.1 / 65.8,
-// 1000 x 200 147 / 131, one query x 100 28.8 / 49.7; d = 16, 1000 x 1000 57.7 / 40.2. One wave per query reading rows lane
-// by lane: d = 128, 2000 x 100 54, 300 x 1000 101.
+//    with every load, 64 lines per instruction, which costs where many rows are read; a slice costs a pass through LDS
+//    each, 30 in a row for d = 960.
+// us per call over 1M rows that no cache holds, rows / slices: d = 128, 100 x 100 21.8 / 23.3, 1000 x 100 29.3 / 28.6,
+// 2000 x 100 39.2 / 37.3, 300 x 300 34.0 / 29.0; d = 96, 2000 x 20 21.1 / 22.5, 1000 x 200 33.8 / 32.0; d = 200, 1000 x 100
+// 38.7 / 34.8, 200 x 1000 65.7 / 53.1, one query x 1000 58.6 / 45.7, 2000 x 20 25.1 / 30.3. In the caches: d = 960, 2000 x 10
+// 37 / 66, one query x 100 29 / 50, 1000 x 200 147 / 131. Rows that are not 16-byte aligned by 4-byte loads: d = 130, 1000 x
+// 100 38.4, by slices of 4-byte loads 52.4. One wave per query reading rows lane by lane: d = 128, 2000 x 100 58.
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -179,12 +180,11 @@ hipError_t launch_rerank(const RerankArgs& a, hipStream_t stream) {
     constexpr int64_t kMaxBlocks = int64_t{1} << 22;
     const int waves = static_cast<int>(a.r < WAVE * kMaxRerankWaves ? (a.r + WAVE - 1) / WAVE : kMaxRerankWaves);
     const dim3 threads(static_cast<unsigned>(waves * WAVE));
-    // Slices where rows are whole halves of lines and a wave takes more than one round of 64 candidates (short rows: more
-    // than one wave's), or where long rows come in numbers that fill the memory's bandwidth.
+    // Slices where a query has many candidates, or more than one wave's and the call gathers 64 MB: there the address
+    // processing counts, below it the latency of the slices' passes through LDS.
     const bool vec4 = a.d % 4 == 0 && reinterpret_cast<uintptr_t>(a.base) % 16 == 0;
-    const bool slices = vec4 && a.d % 16 == 0 &&
-                        (a.r > (a.d <= 32 ? WAVE : WAVE * kMaxRerankWaves) ||
-                         (a.d >= 384 && a.r > WAVE && a.nq >= (int64_t{1} << 24) / (a.r * a.d)));
+    const bool slices = vec4 && a.d >= 16 && a.r > WAVE &&
+                        (a.r > 4 * WAVE || a.nq >= (int64_t{1} << 24) / (a.r * a.d));
     // The slices' buffers also hold the wave lists (K <= 128 pairs a wave); without slices the lists alone.
     const size_t lds = static_cast<size_t>(waves) * (slices ? kSliceBytes : a.K * sizeof(Pair));
     static_assert(2 * WAVE * sizeof(Pair) <= kSliceBytes, "a wave's list fits its slice buffer");
