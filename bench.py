@@ -237,15 +237,16 @@ def bench_ivf(args, centroids, codes, queries, base):
     print(json.dumps(record), flush=True)
 
 
-def load_traffic(cfg, f16):
+def load_traffic(cfg, f16, symbol):
     """Counter record of the search kernel for this configuration (profiles/traffic.json, from rocprofv3 --pmc runs):
-    HBM bytes per launch and the binding pipe, if recorded."""
+    HBM bytes per launch and the binding pipe, if recorded for the kernel that ran (its name `symbol`)."""
     path = os.path.join(ROOT, "profiles", "traffic.json")
     try:
         with open(path) as f:
-            return json.load(f).get(cfg + ("/v9" if f16 else ""))
+            record = json.load(f).get(cfg + ("/v9" if f16 else ""))
     except (OSError, ValueError):
         return None
+    return record if record and record.get("kernel") == symbol else None
 
 
 def main():
@@ -360,25 +361,28 @@ def main():
     q_eff = shape.queries_per_block
     hbm_bytes = float(n) * m * math.ceil(nq / q_eff)
     f16 = variant == vk.ScanVariant.FusedWarpF16
-    # The binding pipe, from the counters of this kernel (profiles/traffic.json): "valu" where the VALU issues more
-    # wave64 instructions per CU-cycle than the LDS is busy (1M and 10M at m=16: 0.91-0.93 against 77-90 %; fp16
-    # tables), "lds" where bank conflicts keep the LDS busier (m=32 and m=64 at k=100, 100M uniform codes: 87-97 %).
-    counters = load_traffic(args.config, f16) or {}
+    # The binding pipe, from the counters of this kernel (profiles/traffic.json; none if another kernel was counted): "valu"
+    # where the VALU issues more wave64 instructions per CU-cycle than the LDS is busy (1M with abandoned tiles 0.92 against
+    # 60 %, 10M 1.01 against 90 %), "lds" where bank conflicts keep the LDS busier (m=32 and m=64 at k=100, 100M uniform
+    # codes: 87-97 %).
+    kernel = s.last_kernel()
+    counters = load_traffic(args.config, f16, kernel.symbol) or {}
     roofline = {
-        "bound": counters.get("bound", "valu"),
+        "bound": counters.get("bound"),
         "bound_basis": ({"valu_instr_per_cu_cycle": counters["valu_per_cu_cycle"], "lds_busy": counters["lds_busy"]}
                         if "lds_busy" in counters else None),
         "achieved": achieved / 1e12,
         "peak": peak / 1e12,
         "unit": "Tlookup/s",
-        "frac": achieved / peak,
+        # A scan that abandons tiles makes only part of the lookups it is counted for: a rate, and no fraction of the peak.
+        "frac": None if kernel.abandons else achieved / peak,
+        "rate_over_peak": achieved / peak,
         "traffic": counters.get("bytes_per_launch"),
         "traffic_detail": counters or None,
-        "kernel": "fused_wave_kernel_t (scan + per-wave top-k)",
+        "kernel": kernel.symbol,
         "kernel_ms": scan_ms,
         "algorithmic": f"n*m*nq = {lookups:.3e} LDS lookups per launch (one {2 if f16 else 4}-byte table read + "
-                       f"one fp32 add each), counted for every vector: scans that abandon tiles make fewer, so the "
-                       f"fraction can exceed 1",
+                       f"one fp32 add each), counted for every vector: scans that abandon tiles make fewer",
         "peak_basis": (f"64 lookups per CU-cycle x {info.sm_count} CUs x {info.clock_khz / 1e6:.2f} GHz: the LDS "
                        f"returns 256 B/clk/CU (one 4-byte fp32 entry per lookup) and the VALU 64 lane-ops/clk/CU "
                        f"(one add, or one v_fma_mix_f32 for fp16 entries, per lookup)"),
@@ -446,7 +450,7 @@ def main():
             "target_frac": 0.80, "achieved_frac": hbm_frac,
             "reason": None if hbm_frac >= 0.80 else
             (f"at Q={q_eff} each code byte serves {q_eff} queries, so the fastest search reads codes at "
-             f"{hbm_frac * 100:.1f} % of the HBM peak while its lookups run at {roofline['frac'] * 100:.1f} % of the "
+             f"{hbm_frac * 100:.1f} % of the HBM peak while its lookups run at {roofline['rate_over_peak'] * 100:.1f} % of the "
              f"lookup peak" + ("" if at_q2 is None else
                                f"; at Q=2 the same search streams codes at {at_q2['frac'] * 100:.1f} % of the HBM peak "
                                f"({at_q2['kernel_ms']:.1f} ms per search against {scan_ms:.1f} ms)")),

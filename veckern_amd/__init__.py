@@ -18,7 +18,7 @@ import numpy as np
 __all__ = [
     "ScanVariant", "Tuning", "Timings", "LaunchShape", "DeviceInfo", "PQSearcher", "VkError",
     "variant_name", "is_fused", "needs_m16", "device_info", "device_count", "dispatched_k", "validate_tuning",
-    "library", "LIB_PATH", "DeviceArray", "Reranker", "IVFIndex", "ivf_assign", "pq_encode", "pq_assign",
+    "library", "LIB_PATH", "DeviceArray", "Reranker", "IVFIndex", "ivf_assign", "pq_encode", "pq_assign", "Abandon", "ScanKernel",
 ]
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
