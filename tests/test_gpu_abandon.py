@@ -151,6 +151,13 @@ def test_abandonment_modes():
             got_d, got_i, _ = s.search(queries, 10, V8)
             assert s.last_kernel().abandons == abandons, (blocks, mode)
             assert_same(got_d, got_i, exp, f"blocks={blocks} mode={mode}")
+        # One query per table earns the first bounds back from 64k vectors per block, unless it is the only slab.
+        s.set_abandon(vk.Abandon.Auto)
+        for count, blocks, abandons in [(4, 3, False), (4, 2, True), (1, 3, True), (1, 5, False)]:
+            s.set_tuning(vk.Tuning(queries_per_block=1, blocks_per_query=blocks))
+            got_d, got_i, _ = s.search(queries[:count], 10, V8)
+            assert s.last_kernel().abandons == abandons, (count, blocks)
+            assert_same(got_d, got_i, exp[:count], f"Q=1 nq={count} blocks={blocks}")
 
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 4097])

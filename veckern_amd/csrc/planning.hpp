@@ -108,11 +108,17 @@ inline bool bulk_scan(const Partition& p, int ilp) {
     return p.grid > 0 && p.total > 0 && block_vectors(p, ilp) < kBulkScanVectors;
 }
 
-// Scans that abandon tiles find bounds first, which a block that scans few vectors does not earn back: at 8-10k vectors
-// per block 43 against 40 us (one query, 1M) and 59 against 58 us (100 queries, 100k), at 39k 64 against 73 us (one
-// query, 10M) and 80 against 111 us (37 queries, 1M). Lists longer than 64 do not use them either: a bound needs more
-// near vectors than a tile holds, and at k = 100 the plain scan was faster (1M, m = 16: 722 against 787 us).
-constexpr int64_t kAbandonVectors = int64_t{1} << 15;
+// Vectors per block from which scans abandon tiles (q queries per table). They find bounds first, which a block that scans
+// few vectors does not earn back. us plain / abandoning on the mixture (1M vectors, m = 16, k = 10), by vectors per block:
+//   Q = 4    8k 70 / 74    12k 81 / 74    16k 82 / 71    31k 95 / 69     36k 97 / 70     83k 128 / 77
+//   Q = 2    8k 48 / 55    20k 59 / 61    24k 62 / 55    31k 60 / 52     43k 70 / 63     83k 88 / 63
+//   Q = 1    8k 42 / 48    24k 53 / 55    36k 54 / 57    56k 61 / 62     67k 70 / 61     83k 83 / 60
+// and m = 32 crosses at 12k to 20k, fp16 tables (Q = 8) below 8k (m = 48 and 64 later, fp16 at 30k and Q <= 2 above 62k, on
+// codes that abandon_pays refuses). One line for all but Q = 1 lies above every crossing; a
+// single query over many blocks, whose scan streams the codes from HBM and reads half of them, takes it too (10M vectors that
+// no cache holds, 39k per block: 73 / 65). Lists longer than 64 do not abandon: a bound needs more near vectors than a tile
+// holds, and at k = 100 the plain scan was faster (1M, m = 16: 722 against 787 us).
+inline int64_t abandon_vectors(int q, int64_t slabs) { return q == 1 && slabs > 1 ? 1 << 16 : 1 << 15; }
 
 // Vectors per block from which the blocks of an abandoning scan (q queries per table) first vote whether it pays. The sample
 // and the plain scan launched after they leave cost 25 us and more, which over fewer vectors is as much as abandoning in vain
@@ -123,7 +129,8 @@ inline int64_t vote_vectors(int q) { return q == 4 ? 1 << 19 : 1 << 18; }
 
 // Whether scans that abandon tiles pay: the mean squared distance between vectors of one tile (past the sort key),
 // against that between vectors far apart in the slot order. Uniform codes have a ratio of 1 and no tile can be dropped;
-// the Gaussian mixture of the benchmark (1000 components, sigma 0.3) about 0.1.
+// the Gaussian mixture of the benchmark (1000 components, sigma 0.3) about 0.2 at m = 16, 0.3 at 32 and 0.75 at 48 and 64. A
+// measure of alikeness and not of the tiles that survive: m = 64 stays plain there, though abandoning took half its time.
 inline bool abandon_pays(double within, double apart) { return within < 0.5 * apart; }
 
 // blocks_x of the unfused scans (searcher.cu:172-177, where the reference also sizes v4 with it): an override, else
