@@ -183,8 +183,8 @@ int vk_search_device(vk_searcher* s, const float* d_queries, size_t nq, size_t k
  * Same arguments, results and errors as vk_search_device for v8_fused_warp and v9_fused_warp_f16 (other variants:
  * VK_ERR_INVALID_ARGUMENT), but the partial lists and slab counters live in a static device array of
  * VK_NOALLOC_SCRATCH_BYTES that the library holds on each device it runs on until the process ends (the first
- * VK_NOALLOC_COUNTER_BYTES for the counters, one 4-byte counter per slab of queries_per_block queries; the rest for
- * the partial lists), so the call makes no device allocation, creates no events and records no timings. A search
+ * VK_NOALLOC_COUNTER_BYTES for the counters, one 4-byte counter per slab of queries_per_block queries, and behind them,
+ * where both fit, one 4-byte bound per query slot for the scan that abandons tiles; the rest for the partial lists), so the call makes no device allocation, creates no events and records no timings. A search
  * needing more than that (very large nq x k) is rejected before any launch with VK_ERR_INVALID_ARGUMENT; split it
  * into smaller calls. The searcher's sorted code layout (v8 and v9) must already exist: one vk_search or
  * vk_search_device call with v8 or v9 builds it (that call allocates); otherwise VK_ERR_LOGIC. Calls on one device

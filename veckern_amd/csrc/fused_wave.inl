@@ -606,8 +606,8 @@ __device__ __forceinline__ bool vote_to_leave(const WaveScanArgs& a, bool leave)
 // IVF (one query per slab, QS = 1): the scan runs over inverted lists. Slab q * a.nprobe + p is the p-th list probed
 // by query q; slabs are in query-major order, so a query's probed lists form one run of consecutive slabs,
 // granules [a.query_gran[q], a.query_gran[q + 1]) of the balanced partition (a.query_gran[nq] = total). Slab s covers
-// the granules from a.query_gran[q] + a.slab_gran[s] to the next slab's start (possibly none), its list's padded tiles start at a.slab_tile[s] in
-// the word-interleaved codes (the plan copies the list's first tile there, one dependent load fewer per slab than
+// the granules from a.query_gran[q] + a.slab_gran[s] to the next slab's start (possibly none), its list's padded tiles
+// start at a.slab_tile[s] in the word-interleaved codes (the plan copies the list's first tile there, one dependent load fewer per slab than
 // looking it up by list), and the vector ids come from a.ids (-1 on padding). A block
 // gathers a query's tables and starts its lists once per run and writes them once, at the end of the run (or of
 // its range); a separate merge kernel combines the partial lists of each query.
@@ -644,8 +644,8 @@ __global__ void __launch_bounds__(T)
     // K real candidates lie at or below it, so nothing beyond it reaches the merged top K; ties at it are kept.
     // In the sorted slot order a tile's vectors are alike, so they fail together: on the 1M-vector Gaussian mixture 98 %
     // of the tiles fail for all four queries after 6 of 16 sub-spaces (65 % after 4), 90 % after 8 of 32.
-    // Measured against the plain scan: 1M x 1000 queries, m = 16, k = 10: 611 -> 308 us (fp16 tables, eight queries: 731
-    // -> 560), 37 queries 110 -> 80 us, one query over 10M 73 -> 64 us.
+    // Measured against the plain scan, inputs changing: 1M x 1000 queries, m = 16, k = 10: 608 -> 329 us (fp16 tables, eight
+    // queries: 728 -> 544), 37 queries 110 -> 80 us, one query over 10M 73 -> 66 us.
     // The first kHeadBytes codes of every vector are read from an array of their own (a.heads): the scan reads half of
     // the code bytes at m = 16 and a quarter at m = 32 .. 64, the rest and the ids only for tiles that are left.
     constexpr bool kPrune = ABANDON;

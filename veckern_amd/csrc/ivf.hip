@@ -29,7 +29,7 @@ constexpr int kMergeThreads = 256;
 constexpr int kPlanThreads = 256;
 constexpr int kScanThreads = 1024;
 // Queries up to which the plan kernel sums the runs itself: every block then writes its XCD's L2 back before it takes
-// the ticket, which over a thousand blocks costs more than the launch it saves.
+// the ticket, which over a thousand blocks costs more than the launch it saves (the figures at vk_ivf::search hold for both).
 constexpr int64_t kTicketQueries = 64;
 
 __device__ __forceinline__ int64_t wave_inclusive_sum(int64_t v) {
